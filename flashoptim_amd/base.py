@@ -581,10 +581,12 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
 
     # ------------------------------------------------------------------------------------ (de)serialisation
     def _state_dict_for_param(self, param_number: int, opt_state: dict[int, Any], hparams: dict[str, Any],
-                              idx_to_param: dict[int, torch.Tensor]) -> dict[str, Any]:
+                              idx_to_param: dict[int, torch.Tensor],
+                              batch: Optional[kernels.ConversionBatch] = None) -> dict[str, Any]:
         """Per-parameter view written to a checkpoint (ref:868-927): quantised states become either their
         codes+scales or a bf16 tensor, and ``error_bits`` is disguised as a tensor of the parameter dtype so
-        that ``Optimizer.load_state_dict``'s cast to the parameter dtype is lossless."""
+        that ``Optimizer.load_state_dict``'s cast to the parameter dtype is lossless.  With a `batch` the converted
+        tensors hold their values once it is launched."""
         out = dict(opt_state[param_number])  # shallow copy: self.state must not change
         if isinstance(out.get("step"), torch.Tensor):
             out["step"] = out["step"].clone()  # live counters may be views into a shared pool
@@ -592,7 +594,7 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
             if name in out:
                 holder = out.pop(name)
                 assert isinstance(holder, _MaybeQuantizedTensor)
-                out.update(holder.state_dict(name=name, allow_quantized=self._compress_state_dict))
+                out.update(holder.state_dict(name=name, allow_quantized=self._compress_state_dict, batch=batch))
         if "error_bits" in out:
             param_dtype = idx_to_param[param_number].dtype
             param_width = _DTYPE_WIDTHS[param_dtype]
@@ -601,7 +603,10 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
             if ecc_width == param_width:
                 out["error_bits"] = errs.view(dtype=param_dtype)          # same width: reinterpret the bits
             elif ecc_width == 1 and param_width == 2:
-                out["error_bits"] = errs.to(dtype=param_dtype)            # int8 -> bf16/fp16 values, exact
+                own = kernels.ConversionBatch() if batch is None else batch
+                out["error_bits"] = own.widen_int8(errs, param_dtype)     # int8 -> bf16/fp16 values, exact
+                if batch is None:
+                    own.launch()
             else:
                 raise NotImplementedError(
                     f"Cannot save {ecc_width}B error correction tensor for {param_width}B parameter. Non-scalar "
@@ -616,11 +621,16 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
         for live, saved in zip(self.param_groups, d["param_groups"]):
             idx_to_param.update(zip(saved["params"], live["params"]))
         state = d["state"]
+        # one launch for the conversions of all parameters; a subclass that writes its parameters in its own way gets
+        # finished tensors from each call instead
+        batch = kernels.ConversionBatch()
+        shared = {"batch": batch} if type(self)._state_dict_for_param is FlashOptimizer._state_dict_for_param else {}
         for group in d["param_groups"]:
             for idx in group["params"]:
                 # torch only lists parameters that already have state
                 if idx in state:
-                    state[idx] = self._state_dict_for_param(idx, state, group, idx_to_param)
+                    state[idx] = self._state_dict_for_param(idx, state, group, idx_to_param, **shared)
+        batch.launch()
         return d
 
     def _load_state_for_param(self, param: torch.Tensor, opt_state: dict[torch.Tensor, Any],

@@ -1,8 +1,11 @@
-// Standalone group codec and ECC kernels for gfx950 with their C entry points: the cold-path companions of
-// the fused step kernels (state initialisation, uncompressed checkpoints, fp32 export/import of master
-// weights).  They share the access shape of the step kernels (fo_device.h) and use correctly rounded division /
-// square root, so that their output equals an IEEE
-// evaluation of the reference formulas operation by operation.
+// Standalone group codec and ECC kernels for gfx950 with their C entry points: the companions of the fused step
+// kernels (state initialisation, checkpoints, fp32 export/import of master weights).  They share the access shape
+// of the step kernels (fo_device.h), and their output equals an IEEE evaluation of the reference formulas operation
+// by operation.
+//
+// All of them only move memory at heart, so each reads its inputs once and writes its result in its final type; and
+// a checkpoint holds hundreds of tensors, most of them short, so the conversions of a whole list share one launch
+// (convert_kernel below).
 //
 // "ref:" cites /root/reference/flashoptim/optimizers.py.
 #include "fo_device.h"
@@ -66,27 +69,117 @@ __device__ const CodeTable<false, true> kCodeTableUS = CodeTable<false, true>();
 __device__ const CodeTable<true, false> kCodeTableS = CodeTable<true, false>();
 __device__ const CodeTable<true, true> kCodeTableSS = CodeTable<true, true>();
 
-// ref:2541-2607 _triton_dequantize_kernel
-template <bool FAST>
-__device__ __forceinline__ void dequantize_load(const void* codes, const uint16_t* scales, int64_t first, int64_t n,
-                                                Pack<1, 4>& craw, uint16_t& scale_bits) {
-    load_lane<1, 4, FAST>(craw, codes, first, n);
-    scale_bits = 0x3c00;                                                    // ref:2577-2582 masked scales read 1.0
-    if (FAST || first < n) scale_bits = scales[first >> 5];
-}
-template <bool FAST>
-__device__ __forceinline__ void dequantize_finish(const Pack<1, 4>& craw, uint16_t scale_bits, const float* lut, float* out,
-                                                  int64_t first, int64_t n, CodecFlags f) {
-    const float scale = f16_bits_to_f32(scale_bits);
-    Pack<4, 4> o;
+// ------------------------------------------------------------------------------------------------
+// one launch over a list of tensors
+// ------------------------------------------------------------------------------------------------
+
+// The list travels as the kernel's argument (3.3 KiB of the 4 KiB a launch may pass): no table is uploaded and no
+// memory has to outlive the call.  A workgroup (one wavefront) finds its job with one vector load and a ballot: lane l
+// reads where job l's workgroups start, the number of lanes that start at or before this workgroup names the job.
+constexpr int kJobsPerLaunch = 64;
+struct JobBatch {
+    fo_convert_job job[kJobsPerLaunch];
+    u32 first_block[kJobsPerLaunch];
+    int32_t count, reserved;
+};
+static_assert(sizeof(JobBatch) <= 3584, "a batch must fit the kernel argument segment");
+
+// Op: kEpl elements per lane and span, kSpans neighbouring spans of 64 * kEpl elements per workgroup; a Raw holds
+// what a lane has loaded for one span; all loads of a workgroup are issued before the first span is finished.
+template <class Op> struct ConvertShape {
+    static constexpr int64_t kSpan = 64 * Op::kEpl;
+    static constexpr int64_t kBlock = kSpan * Op::kSpans;
+};
+
+template <class Op, int MODE>
+__device__ __forceinline__ void convert_block(const fo_convert_job& job, int64_t base, float* lut) {
+    typename Op::Raw raw[Op::kSpans];
+    const int lane = (int)threadIdx.x * Op::kEpl;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        float xv = lut[byte_of<4>(craw, k)] * scale;                        // ref:2591-2600
-        if (f.do_sqrt) xv = xv * xv;                                        // ref:2603-2604
-        o.w[k] = as_u32(xv);
-    }
-    store_lane<4, 4, FAST>(o, out, first, n);
+    for (int i = 0; i < Op::kSpans; ++i) Op::template load<MODE>(job, Where{base + i * ConvertShape<Op>::kSpan, lane}, raw[i]);
+    Op::prepare(job, lut);
+#pragma unroll
+    for (int i = 0; i < Op::kSpans; ++i) Op::template finish<MODE>(job, Where{base + i * ConvertShape<Op>::kSpan, lane}, raw[i], lut);
 }
+
+template <class Op> __global__ __launch_bounds__(kCodecThreads) void convert_kernel(JobBatch b) {
+    __shared__ __align__(16) float lut[Op::kLutFloats];
+    const u32 start = (int)threadIdx.x < b.count ? b.first_block[threadIdx.x] : 0xffffffffu;
+    const int j = __builtin_popcountll(__builtin_amdgcn_ballot_w64(start <= blockIdx.x)) - 1;  // job 0 starts at 0
+    const fo_convert_job job = b.job[j];
+    const int64_t base = (int64_t)(blockIdx.x - b.first_block[j]) * ConvertShape<Op>::kBlock;
+    // workgroup-uniform choice of the access mode
+    if (!Op::aligned(job)) convert_block<Op, kGuarded>(job, base, lut);
+    else if (base + ConvertShape<Op>::kBlock <= job.n) convert_block<Op, kVector>(job, base, lut);
+    else convert_block<Op, kLane>(job, base, lut);
+}
+
+__device__ __forceinline__ bool aligned16(const void* a, const void* b) { return (((uintptr_t)a | (uintptr_t)b) & 15u) == 0; }
+
+// x where it is a number, the quiet NaN 0x7fc00000 otherwise: in front of a conversion to bf16 the result then has the
+// bits of torch's cast, which writes 0x7fc0 for every NaN (the conversion instruction keeps sign and payload; for fp16
+// the cast does so too).
+template <int DT> __device__ __forceinline__ float one_nan(float x) { return (DT == DT_BF16 && x != x) ? as_f32(0x7fc00000u) : x; }
+
+// ref:2541-2607 _triton_dequantize_kernel, with the cast to the output type that follows it in a checkpoint (ref:167).
+// Bound by memory: 1.06 bytes in and 4 (fp32) or 2 (bf16) out per element.  kSpans: the 1 KiB table that a workgroup
+// copies to LDS serves 1024 (fp32) or 2048 (bf16) elements; with one span per workgroup fp32 reached 4.7 instead of
+// 5.6 TB/s, reading the table through the vector cache instead 3.5.  An AdamW checkpoint of 2.2e8 weights (bf16, 24-bit
+// masters; this kernel and Int8WidenOp) takes 315 us, 6.3 TB/s, where fp32 values, their casts and torch's int8 cast
+// (1.3 TB/s) took 1456.
+template <int ODT> struct DequantizeOp {
+    static constexpr int kEpl = DTypeInfo<ODT>::epl, kSpans = 4, kLutFloats = 256;
+    struct Raw { Pack<1, kEpl> codes; uint16_t scale; };
+    __device__ __forceinline__ static bool aligned(const fo_convert_job& j) { return aligned16(j.src, j.dst); }
+    template <int MODE> __device__ __forceinline__ static void load(const fo_convert_job& j, Where w, Raw& r) {
+        load_lane<1, kEpl, MODE>(r.codes, j.src, w, j.n);
+        r.scale = 0x3c00;                                                   // ref:2577-2582 masked scales read 1.0
+        if (MODE == kVector || w.first() < j.n) r.scale = load_scale(static_cast<const uint16_t*>(j.src2), w);
+    }
+    __device__ __forceinline__ static void prepare(const fo_convert_job& j, float* lut) {
+        const bool is_signed = j.flags & FO_CODEC_SIGNED, softsign = j.flags & FO_CODEC_SOFTSIGN;
+        const float* table = is_signed ? (softsign ? kCodeTableSS.v : kCodeTableS.v) : (softsign ? kCodeTableUS.v : kCodeTableU.v);
+        *reinterpret_cast<u32x4*>(lut + 4 * threadIdx.x) = *reinterpret_cast<const u32x4*>(table + 4 * threadIdx.x);
+        __syncthreads();  // one wavefront: no hardware barrier is needed, the compiler drops it
+    }
+    template <int MODE> __device__ __forceinline__ static void finish(const fo_convert_job& j, Where w, Raw& r, const float* lut) {
+        const float scale = f16_bits_to_f32(r.scale);
+        float x[kEpl];
+#pragma unroll
+        for (int k = 0; k < kEpl; ++k) {
+            x[k] = lut[byte_of<kEpl>(r.codes, k)] * scale;                  // ref:2591-2600
+            if (j.flags & FO_CODEC_SQRT) x[k] = x[k] * x[k];                // ref:2603-2604
+        }
+        Pack<DTypeInfo<ODT>::bytes, kEpl> o;
+#pragma unroll
+        for (int k = 0; k < kEpl; k += 2) {
+            float wa, wb;
+            narrow_pair<ODT, kEpl>(o, k, one_nan<ODT>(x[k]), one_nan<ODT>(x[k + 1]), wa, wb);
+        }
+        store_lane<DTypeInfo<ODT>::bytes, kEpl, MODE>(o, j.dst, w, j.n);
+    }
+};
+
+// int8 codes as values of a 2-byte type (exact): the form in which a checkpoint holds 1-byte correction codes
+// (ref:900-927).  One byte in, two out.
+template <int DT> struct Int8WidenOp {
+    static constexpr int kEpl = 8, kSpans = 4, kLutFloats = 4;
+    struct Raw { Pack<1, 8> codes; };
+    __device__ __forceinline__ static bool aligned(const fo_convert_job& j) { return aligned16(j.src, j.dst); }
+    template <int MODE> __device__ __forceinline__ static void load(const fo_convert_job& j, Where w, Raw& r) {
+        load_lane<1, 8, MODE>(r.codes, j.src, w, j.n);
+    }
+    __device__ __forceinline__ static void prepare(const fo_convert_job&, float*) {}
+    template <int MODE> __device__ __forceinline__ static void finish(const fo_convert_job& j, Where w, Raw& r, const float*) {
+        Pack<2, 8> o;
+#pragma unroll
+        for (int k = 0; k < 8; k += 2) {
+            float wa, wb;
+            narrow_pair<DT, 8>(o, k, ecc_to_float<1, 8>(r.codes, k), ecc_to_float<1, 8>(r.codes, k + 1), wa, wb);
+        }
+        store_lane<2, 8, MODE>(o, j.dst, w, j.n);
+    }
+};
 
 // ref:2779-2803 _reconstruct_fp32_kernel
 template <int DT, int ECCB, bool FAST>
@@ -118,7 +211,7 @@ __device__ __forceinline__ void ecc_split_lane(const float* x, const void* narro
     store_lane<ECCB, EPL, FAST>(eout, ecc, first, n);
 }
 
-// Work loop shared by the four kernels, in the step kernels' geometry: a workgroup is one wavefront and takes one
+// Work loop shared by the kernels over one tensor, in the step kernels' geometry: a workgroup is one wavefront and takes one
 // span of 64 x EPL elements (it only iterates for tensors beyond 2^31 - 1 spans); `first` is the lane's first element.
 #define FO_SPAN_LOOP(N, EPL_, ALIGNED, CALL_FAST, CALL_SLOW)                                      \
     {                                                                                             \
@@ -134,45 +227,6 @@ template <int XDT>
 __global__ __launch_bounds__(kCodecThreads) void quantize_kernel(const void* x, void* codes, uint16_t* scales, int64_t n, CodecFlags f) {
     const bool aligned = ((((uintptr_t)x) | ((uintptr_t)codes)) & 15u) == 0;
     FO_SPAN_LOOP(n, DTypeInfo<XDT>::epl, aligned, (quantize_lane<XDT, true>(x, codes, scales, first, n, f)), (quantize_lane<XDT, false>(x, codes, scales, first, n, f)))
-}
-
-// A workgroup (one wavefront) takes kDequantSpans neighbouring spans of 256 elements, so that the 1 KiB table it
-// copies to LDS serves more than one span (4 spans: 5.6 TB/s, 1 span: 4.7; reading the table through the vector
-// cache instead: 3.5); all code loads are issued before the table is committed.  Four of every five bytes are
-// written, and write-only streams reach 5.7-6.0 TB/s on this part.
-constexpr int kDequantSpans = 4;
-__global__ __launch_bounds__(kCodecThreads) void dequantize_kernel(const void* codes, const uint16_t* scales, float* out, int64_t n, CodecFlags f) {
-    constexpr int kSpans = kDequantSpans;
-    constexpr int64_t kSpan = 64 * 4;
-    const bool aligned = ((((uintptr_t)out) | ((uintptr_t)codes)) & 15u) == 0;
-    const float* table = f.is_signed ? (f.softsign ? kCodeTableSS.v : kCodeTableS.v) : (f.softsign ? kCodeTableUS.v : kCodeTableU.v);
-    __shared__ __align__(16) float lut[256];
-    const u32x4 frag = *reinterpret_cast<const u32x4*>(table + 4 * threadIdx.x);
-    bool committed = false;
-    const int64_t n_blocks = (n + kSpan * kSpans - 1) / (kSpan * kSpans);
-    for (int64_t blk = blockIdx.x; blk < n_blocks; blk += gridDim.x) {
-        const int64_t base = blk * kSpan * kSpans;
-        const bool fast = aligned && base + kSpan * kSpans <= n;
-        Pack<1, 4> craw[kSpans];
-        uint16_t scale_bits[kSpans];
-#pragma unroll
-        for (int i = 0; i < kSpans; ++i) {
-            const int64_t first = base + i * kSpan + (int64_t)threadIdx.x * 4;
-            if (fast) dequantize_load<true>(codes, scales, first, n, craw[i], scale_bits[i]);
-            else dequantize_load<false>(codes, scales, first, n, craw[i], scale_bits[i]);
-        }
-        if (!committed) {
-            *reinterpret_cast<u32x4*>(lut + 4 * threadIdx.x) = frag;
-            __syncthreads();  // one wavefront: no hardware barrier is needed, the compiler drops it
-            committed = true;
-        }
-#pragma unroll
-        for (int i = 0; i < kSpans; ++i) {
-            const int64_t first = base + i * kSpan + (int64_t)threadIdx.x * 4;
-            if (fast) dequantize_finish<true>(craw[i], scale_bits[i], lut, out, first, n, f);
-            else dequantize_finish<false>(craw[i], scale_bits[i], lut, out, first, n, f);
-        }
-    }
 }
 
 template <int DT, int ECCB>
@@ -196,6 +250,51 @@ using namespace fo_host;
 unsigned grid_for(int64_t n, int epl) {
     const int64_t spans = (n + 64 * epl - 1) / (64 * epl);
     return (unsigned)(spans < INT32_MAX ? spans : INT32_MAX);
+}
+
+// Enqueues the jobs, kJobsPerLaunch to a launch; the caller has checked their pointers.
+template <class Op> int launch_jobs(const fo_convert_job* jobs, int64_t n_jobs, hipStream_t stream) {
+    fo::JobBatch b;
+    b.count = 0; b.reserved = 0;
+    int64_t blocks = 0;
+    const auto flush = [&]() -> int {
+        if (b.count == 0) return 0;
+        hipLaunchKernelGGL(fo::convert_kernel<Op>, dim3((unsigned)blocks), dim3(fo::kCodecThreads), 0, stream, b);
+        b.count = 0; blocks = 0;
+        return check_hip(hipGetLastError(), "conversion kernel launch");
+    };
+    for (int64_t i = 0; i < n_jobs; ++i) {
+        if (jobs[i].n == 0) continue;
+        const int64_t need = (jobs[i].n + fo::ConvertShape<Op>::kBlock - 1) / fo::ConvertShape<Op>::kBlock;
+        if (need > INT32_MAX) return fail(FO_ERR_INVALID_ARGUMENT, "tensor too large for one launch (%lld elements)", (long long)jobs[i].n);
+        if (b.count == fo::kJobsPerLaunch || blocks + need > INT32_MAX)
+            if (int rc = flush()) return rc;
+        b.job[b.count] = jobs[i];
+        b.first_block[b.count++] = (fo::u32)blocks;
+        blocks += need;
+    }
+    return flush();
+}
+
+// What every job list has to satisfy before a kernel sees its pointers: src, dst (and src2, dst2 where the kernel uses
+// them) are there, each aligned to `*_align` bytes.  An align of 0 is an unused pointer.
+int validate_jobs(const fo_convert_job* jobs, int64_t n_jobs, unsigned src_align, unsigned src2_align, unsigned dst_align, unsigned dst2_align) {
+    if (n_jobs < 0) return fail(FO_ERR_INVALID_ARGUMENT, "negative job count");
+    if (n_jobs > 0 && !jobs) return fail(FO_ERR_INVALID_ARGUMENT, "jobs must not be NULL");
+    for (int64_t i = 0; i < n_jobs; ++i) {
+        const fo_convert_job& j = jobs[i];
+        if (j.n < 0) return fail(FO_ERR_INVALID_ARGUMENT, "n must be >= 0");
+        if (j.n == 0) continue;
+        const void* p[4] = {j.src, j.src2, j.dst, j.dst2};
+        const unsigned align[4] = {src_align, src2_align, dst_align, dst2_align};
+        for (int k = 0; k < 4; ++k) {
+            if (!align[k]) continue;
+            if (!p[k]) return fail(FO_ERR_INVALID_ARGUMENT, "job %lld: pointers must not be NULL", (long long)i);
+            if ((uintptr_t)p[k] & (align[k] - 1)) return fail(FO_ERR_INVALID_ARGUMENT, "job %lld: pointer not aligned to its element size", (long long)i);
+        }
+    }
+    if (n_jobs > 0 && compute_units() <= 0) return fail(FO_ERR_NO_DEVICE, "no HIP device");
+    return 0;
 }
 
 }  // namespace
@@ -227,11 +326,23 @@ int fo_dequantize(const void* codes, const void* scales, float* out, int64_t n, 
     if (n == 0) return 0;  // ref:2533
     if (!codes || !scales || !out) return fail(FO_ERR_INVALID_ARGUMENT, "codes, scales and out must not be NULL");
     if (((uintptr_t)out & 3) || ((uintptr_t)scales & 1)) return fail(FO_ERR_INVALID_ARGUMENT, "out or scales not aligned to their element size");
-    if (compute_units() <= 0) return fail(FO_ERR_NO_DEVICE, "no HIP device");
-    const fo::CodecFlags f{is_signed ? 1 : 0, do_sqrt ? 1 : 0, softsign ? 1 : 0};
-    hipLaunchKernelGGL(fo::dequantize_kernel, dim3(grid_for(n, 4 * fo::kDequantSpans)), dim3(fo::kCodecThreads), 0, (hipStream_t)stream, codes,
-                       (const uint16_t*)scales, out, n, f);
-    return check_hip(hipGetLastError(), "dequantize kernel launch");
+    const int32_t flags = (is_signed ? FO_CODEC_SIGNED : 0) | (do_sqrt ? FO_CODEC_SQRT : 0) | (softsign ? FO_CODEC_SOFTSIGN : 0);
+    const fo_convert_job job{codes, scales, out, nullptr, n, flags, 0};
+    return fo_dequantize_many(&job, 1, FO_F32, stream);
+}
+
+int fo_dequantize_many(const fo_convert_job* jobs, int64_t n_jobs, int out_dtype, void* stream) {
+    if (out_dtype != FO_F32 && out_dtype != FO_BF16) return fail(FO_ERR_INVALID_ARGUMENT, "output dtype must be fp32 or bf16 (got %d)", out_dtype);
+    if (int rc = validate_jobs(jobs, n_jobs, 1, 2, out_dtype == FO_F32 ? 4 : 2, 0)) return rc;
+    return out_dtype == FO_F32 ? launch_jobs<fo::DequantizeOp<fo::DT_F32>>(jobs, n_jobs, (hipStream_t)stream)
+                               : launch_jobs<fo::DequantizeOp<fo::DT_BF16>>(jobs, n_jobs, (hipStream_t)stream);
+}
+
+int fo_int8_widen_many(const fo_convert_job* jobs, int64_t n_jobs, int dtype, void* stream) {
+    if (dtype != FO_BF16 && dtype != FO_F16) return fail(FO_ERR_INVALID_ARGUMENT, "dtype must be bf16 or fp16 (got %d)", dtype);
+    if (int rc = validate_jobs(jobs, n_jobs, 1, 0, 2, 0)) return rc;
+    return dtype == FO_BF16 ? launch_jobs<fo::Int8WidenOp<fo::DT_BF16>>(jobs, n_jobs, (hipStream_t)stream)
+                            : launch_jobs<fo::Int8WidenOp<fo::DT_F16>>(jobs, n_jobs, (hipStream_t)stream);
 }
 
 static int validate_ecc_args(const void* a, const void* b, const void* c, int narrow_dtype, int ecc_bytes, int64_t n) {

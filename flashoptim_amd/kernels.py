@@ -9,6 +9,7 @@ All of them are asynchronous on the current stream of the tensors' device and mu
 
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
@@ -95,6 +96,17 @@ def quantize(
     return out_int8, out_scales
 
 
+def _check_codes(codes: torch.Tensor, scales: torch.Tensor, signed: bool) -> None:
+    _require_device(codes, "dequantize")
+    if codes.dtype != (torch.int8 if signed else torch.uint8):
+        raise ValueError(f"codes must be {'int8' if signed else 'uint8'} for signed={signed}, got {codes.dtype}.")
+    if scales.dtype != torch.float16:
+        raise ValueError(f"scales must be fp16, got {scales.dtype}.")
+    if scales.numel() < (codes.numel() + GROUP_SIZE - 1) // GROUP_SIZE:
+        raise ValueError("too few scales for the number of codes")
+    _require_same_device(codes, scales, "in_scales")
+
+
 def dequantize(
     in_int8: torch.Tensor,
     in_scales: torch.Tensor,
@@ -106,21 +118,14 @@ def dequantize(
 ) -> torch.Tensor:
     """Inverse of :func:`quantize`; returns fp32 with the shape of the codes (ref:2529-2538)."""
     _check_group_size(group_size)
-    _require_device(in_int8, "dequantize")
-    if in_int8.dtype != (torch.int8 if signed else torch.uint8):
-        raise ValueError(f"codes must be {'int8' if signed else 'uint8'} for signed={signed}, got {in_int8.dtype}.")
-    if in_scales.dtype != torch.float16:
-        raise ValueError(f"scales must be fp16, got {in_scales.dtype}.")
+    _check_codes(in_int8, in_scales, signed)
     codes = in_int8 if in_int8.is_contiguous() else in_int8.contiguous()
     scales = in_scales if in_scales.is_contiguous() else in_scales.contiguous()
     n = codes.numel()
-    if scales.numel() < (n + GROUP_SIZE - 1) // GROUP_SIZE:
-        raise ValueError("too few scales for the number of codes")
     if out_float is None:
         out_float = torch.empty_like(codes, dtype=torch.float32)
     if out_float.dtype != torch.float32 or out_float.numel() != n or not out_float.is_contiguous():
         raise ValueError("out_float must be a contiguous fp32 tensor with as many elements as the codes")
-    _require_same_device(codes, scales, "in_scales")
     _require_same_device(codes, out_float, "out_float")
     if n > 0:
         with _native.device_guard(codes.device):
@@ -130,6 +135,60 @@ def dequantize(
             )
         _native.check(rc, "fo_dequantize")
     return out_float
+
+
+# --------------------------------------------------------------------------- conversions of many tensors
+
+_CODEC_SIGNED, _CODEC_SQRT, _CODEC_SOFTSIGN = 1, 2, 4  # fo_codec_flags
+
+
+class ConversionBatch:
+    """Conversions of many tensors, issued as one launch per kind, dtype and device (up to 64 tensors each) instead of
+    one or two launches per tensor.
+
+    A method allocates its output and returns it at once; the values are there, in stream order, after ``launch()``.
+    A batch is used by one thread, inside one call of this package.
+    """
+
+    def __init__(self) -> None:
+        self._jobs: dict = {}  # (entry point, *its leading arguments, device) -> flat list of fo_convert_job words
+        self._keepalive: list = []  # inputs must outlive the launch
+
+    def _add(self, entry: tuple, device: torch.device, src: torch.Tensor, src2, dst: torch.Tensor, dst2, flags: int = 0) -> None:
+        ptr = _native.ptr
+        self._jobs.setdefault((entry, device), []).extend(
+            (src.data_ptr(), ptr(src2) or 0, dst.data_ptr(), ptr(dst2) or 0, dst.numel(), flags))
+        self._keepalive.append((src, src2, dst, dst2))
+
+    def dequantize_bf16(self, codes: torch.Tensor, scales: torch.Tensor, signed: bool, sqrt: bool, softsign: bool) -> torch.Tensor:
+        """``dequantize(codes, scales, ...).to(torch.bfloat16)``."""
+        _check_codes(codes, scales, signed)
+        codes, scales = codes.contiguous(), scales.contiguous()
+        out = torch.empty_like(codes, dtype=torch.bfloat16)
+        if codes.numel() > 0:
+            flags = (_CODEC_SIGNED if signed else 0) | (_CODEC_SQRT if sqrt else 0) | (_CODEC_SOFTSIGN if softsign else 0)
+            self._add(("fo_dequantize_many", DTYPE_CODE[torch.bfloat16]), codes.device, codes, scales, out, None, flags)
+        return out
+
+    def widen_int8(self, values: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+        """``values.to(dtype)`` of an int8 tensor, dtype bf16 or fp16."""
+        if (type(values) is not torch.Tensor or not values.is_cuda or values.dtype != torch.int8
+                or not values.is_contiguous() or dtype not in (torch.bfloat16, torch.float16)):
+            return values.to(dtype=dtype)
+        out = torch.empty_like(values, dtype=dtype)
+        if values.numel() > 0:
+            self._add(("fo_int8_widen_many", DTYPE_CODE[dtype]), values.device, values, None, out, None)
+        return out
+
+    def launch(self) -> None:
+        """Enqueue everything collected so far on the current stream of each device."""
+        jobs, self._jobs = self._jobs, {}
+        for ((name, *args), device), words in jobs.items():
+            table = (ctypes.c_int64 * len(words))(*words)
+            with _native.device_guard(device):
+                rc = getattr(_native.lib(), name)(table, len(words) // 6, *args, _native.current_stream_ptr(device))
+            _native.check(rc, name)
+        self._keepalive.clear()
 
 
 # ------------------------------------------------------------------------------------------------- ECC

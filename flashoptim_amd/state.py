@@ -13,7 +13,7 @@ from typing import Optional
 
 import torch
 
-from .kernels import dequantize, quantize
+from .kernels import ConversionBatch, dequantize, quantize
 
 QUANTIZED_SUFFIX = "::quantized"
 SCALES_SUFFIX = "::scales"
@@ -156,12 +156,19 @@ class _MaybeQuantizedTensor:
     def _quantized_scales_key(name: str) -> str:
         return name + SCALES_SUFFIX
 
-    def state_dict(self, name: str, allow_quantized: bool = False) -> dict[str, torch.Tensor]:
+    def state_dict(self, name: str, allow_quantized: bool = False,
+                   batch: Optional[ConversionBatch] = None) -> dict[str, torch.Tensor]:
         """``{name::quantized, name::scales}`` for a compressed checkpoint, else ``{name: bf16 tensor}`` which a
-        stock torch optimizer can load (ref:159-167)."""
-        if allow_quantized and self.is_quantized():
+        stock torch optimizer can load (ref:159-167).  With a `batch` the bf16 values are there once it is launched."""
+        if not self.is_quantized():
+            return {name: self.data.to(dtype=torch.bfloat16)}
+        if allow_quantized:
             return {self._quantized_vals_key(name): self.quantized, self._quantized_scales_key(name): self.scales}
-        return {name: self.materialize().to(dtype=torch.bfloat16)}
+        own = ConversionBatch() if batch is None else batch
+        out = own.dequantize_bf16(self.quantized, self.scales, self._signed, self._sqrt, self._softsign)
+        if batch is None:
+            own.launch()
+        return {name: out}
 
     def load_state_dict(self, d: dict[str, torch.Tensor], name: str) -> None:
         """Accepts the whole per-parameter state dict; only ``name`` and ``name::*`` are looked at (ref:191-210)."""

@@ -1,0 +1,64 @@
+"""The conversions of checkpoints and fp32 import/export over lists of tensors (csrc/fo_codec.hip: convert_kernel),
+against the oracle or the eager sequence they stand for.  Every value is exact: the same IEEE operations, one rounding to
+the output type."""
+
+import pytest
+import torch
+
+from oracle import c_oracle as C
+from tests import parity
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+# lanes, spans and workgroups of every kernel end at these lengths (8 / 4 elements, 512 / 256, 2048 / 1024), and around them
+LENGTHS = [1, 7, 8, 9, 31, 33, 255, 257, 511, 512, 513, 1023, 1025, 2047, 2048, 2049, 4097, 70001]
+
+
+def _lengths(many: bool):
+    """`many`: more tensors than one launch takes, an empty one among them."""
+    return LENGTHS + ([0] + [3 * i + 1 for i in range(90)] if many else [])
+
+
+def _at(values: torch.Tensor, offset: int) -> torch.Tensor:
+    """`values` on the GPU, `offset` elements into a larger buffer (offset 1: no vector access is aligned)."""
+    buf = torch.zeros(values.numel() + offset, dtype=values.dtype, device=DEV)
+    buf[offset:].copy_(values)
+    return buf[offset:]
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("signed,sqrt,softsign", [(True, False, True), (False, True, False), (True, True, False), (False, False, True)])
+def test_dequantize_to_bf16_over_a_list(signed, sqrt, softsign, offset):
+    from flashoptim_amd.kernels import ConversionBatch, dequantize
+
+    g = torch.Generator().manual_seed(5)
+    batch, cases = ConversionBatch(), []
+    for n in _lengths(many=offset == 0):
+        codes = torch.randint(0, 256, (n,), generator=g, dtype=torch.int32).to(torch.uint8)
+        codes = codes.view(torch.int8) if signed else codes
+        scales = torch.randn((n + 31) // 32, generator=g).abs().to(torch.float16)
+        if n > 512:
+            scales[1], codes[33] = float("inf"), 0  # inf * 0
+        dev = _at(codes, offset), scales.to(DEV)
+        cases.append((codes, scales, dev, batch.dequantize_bf16(*dev, signed, sqrt, softsign)))
+    batch.launch()
+    for codes, scales, dev, got in cases:
+        eager = dequantize(*dev, signed=signed, sqrt=sqrt, softsign=softsign).to(torch.bfloat16)
+        assert torch.equal(got.view(torch.int16), eager.view(torch.int16)), codes.numel()  # NaN bits too
+        ref = C.dequantize(codes, scales, signed, sqrt, softsign).to(torch.bfloat16)
+        assert torch.equal(got.cpu().nan_to_num(7.0), ref.nan_to_num(7.0)), codes.numel()  # a CPU's own NaN has a sign
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_widen_int8_over_a_list(dtype, offset):
+    from flashoptim_amd.kernels import ConversionBatch
+
+    batch, cases = ConversionBatch(), []
+    for n in _lengths(many=offset == 0):
+        values = (torch.arange(n) * 37 % 256 - 128).to(torch.int8)
+        cases.append((values, batch.widen_int8(_at(values, offset), dtype)))
+    batch.launch()
+    for values, got in cases:
+        assert parity.bits_equal(got, values.to(dtype)), values.numel()

@@ -634,8 +634,9 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
         return d
 
     def _load_state_for_param(self, param: torch.Tensor, opt_state: dict[torch.Tensor, Any],
-                              hparams: dict[str, Any]) -> dict[str, Any]:
-        """Inverse of :meth:`_state_dict_for_param` on the already dtype-cast tensors (ref:797-866)."""
+                              hparams: dict[str, Any], batch: Optional[kernels.ConversionBatch] = None) -> dict[str, Any]:
+        """Inverse of :meth:`_state_dict_for_param` on the already dtype-cast tensors (ref:797-866).  With a `batch`
+        the converted tensors hold their values once it is launched."""
         saved = opt_state[param]
         spec = self._quantized_state_spec()
         restored = {k: v for k, v in saved.items() if not any(k == q or k.startswith(q + "::") for q in spec)}
@@ -644,7 +645,7 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
             if any(k.startswith(name) for k in saved):
                 restored[name] = _MaybeQuantizedTensor.from_state_dict(
                     saved, name=name, try_quantize=quantize, signed=s.signed, sqrt=s.sqrt, softsign=s.softsign,
-                    storage_dtype=param.dtype,
+                    storage_dtype=param.dtype, batch=batch,
                 )
         master_bytewidth = hparams.get("master_bytewidth")
         if master_bytewidth is None:
@@ -656,7 +657,10 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
         ecc_width = int(master_bytewidth) - param_width
         seen_dtype = errs.dtype
         if ecc_width == 1 and errs.dtype != torch.int8:
-            errs = errs.to(dtype=torch.int8)
+            own = kernels.ConversionBatch() if batch is None else batch
+            errs = own.narrow_to_int8(errs)
+            if batch is None:
+                own.launch()
         elif ecc_width == 2 and errs.dtype != torch.int16:
             errs = errs.view(dtype=torch.int16)
         if param_width + _DTYPE_WIDTHS[errs.dtype] != int(master_bytewidth):
@@ -690,15 +694,19 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
             self._state_ready = set()
             return
         opt_state = cast(dict[torch.Tensor, Any], state["state"])
+        # one launch for the conversions of all parameters, as in state_dict()
+        batch = kernels.ConversionBatch()
+        shared = {"batch": batch} if type(self)._load_state_for_param is FlashOptimizer._load_state_for_param else {}
         for group in cast(list[dict[str, Any]], state["param_groups"]):
             for param in group["params"]:
                 per_param = opt_state[param]
                 for k, v in per_param.items():
                     if isinstance(v, torch.Tensor):
                         per_param[k] = self._get_local_tensor(v)
-                opt_state[param] = self._load_state_for_param(param, opt_state, hparams=group)
+                opt_state[param] = self._load_state_for_param(param, opt_state, hparams=group, **shared)
             # after the per-parameter pass, so that a master_bytewidth found there is known to come from the file
             group.setdefault("master_bytewidth", self._master_bytewidth)
+        batch.launch()
         super().__setstate__(state)
         # state tensors were replaced: cached pointer tables and step counters are stale
         self._plan_epoch = getattr(self, "_plan_epoch", 0) + 1

@@ -16,40 +16,6 @@ namespace fo {
 
 constexpr int kCodecThreads = 64;   // one wavefront per workgroup, like the step kernels
 
-struct CodecFlags {
-    int is_signed, do_sqrt, softsign;
-};
-
-// ref:2610-2676 _triton_quantize_kernel
-template <int XDT, bool FAST>
-__device__ __forceinline__ void quantize_lane(const void* x, void* codes, uint16_t* scales, int64_t first, int64_t n, CodecFlags f) {
-    constexpr int EPL = DTypeInfo<XDT>::epl;
-    Pack<DTypeInfo<XDT>::bytes, EPL> xraw;
-    load_lane<DTypeInfo<XDT>::bytes, EPL, FAST>(xraw, x, first, n);
-    float v[EPL];
-    float am = 0.0f;
-#pragma unroll
-    for (int k = 0; k < EPL; ++k) {
-        float t = widen<XDT, EPL>(xraw, k);
-        if (f.do_sqrt) t = sqrt_rn(t);                                      // ref:2650-2651
-        v[k] = t;
-        am = fmaxf(am, fabsf(t));
-    }
-    am = fmaxf(group_max<EPL>(am), 1e-12f);                                 // ref:2657-2658
-    const float out_max = f.is_signed ? 127.0f : 255.0f;
-    u32 q[EPL];
-#pragma unroll
-    for (int k = 0; k < EPL; ++k) {
-        const float nrm = div_rn(v[k], am);                                 // ref:2661
-        const float t = f.softsign ? div_rn(2.0f * nrm, 1.0f + fabsf(nrm)) : nrm;   // ref:2664-2667
-        q[k] = (u32)(int)floorf(t * out_max + 0.5f);                        // ref:2670-2671
-    }
-    Pack<1, EPL> out;
-    pack_codes<1, EPL>(q, out);
-    store_lane<1, EPL, FAST>(out, codes, first, n);
-    if ((FAST || first < n) && (threadIdx.x & (32 / EPL - 1)) == 0) store_scale(scales, first >> 5, f32_to_f16_bits(am));   // ref:2675-2676
-}
-
 // Value of code byte b before the group scale: q / IN_MAX, then y / (2 - |y|) when the softsign companding is on
 // (ref:2591-2597), each operation correctly rounded.  Evaluated by the compiler, one table per flag combination;
 // a lookup replaces two IEEE divisions per element.
@@ -160,6 +126,84 @@ template <int ODT> struct DequantizeOp {
     }
 };
 
+// One span of values as the verified flow sees it from a lane (fo_math.h: codec_verified).
+template <int EPL> struct CodecLane {
+    const float (&v)[EPL];
+    float am;
+    Pack<1, EPL>& out;
+    float x[EPL], slack[EPL], least;
+    __device__ __forceinline__ void convert(const float (&q)[EPL]) {
+        if constexpr (EPL == 8) {
+            const float lo[4] = {q[0], q[1], q[2], q[3]}, hi[4] = {q[4], q[5], q[6], q[7]};
+            convert_pack8<kFloor, kFloor>(lo, hi, out.w[0], out.w[1]);
+        } else {
+            u32 c[EPL];
+#pragma unroll
+            for (int k = 0; k < EPL; ++k) c[k] = (u32)hw::floor_to_int(q[k]);
+            pack_codes<1, EPL>(c, out);
+        }
+    }
+    __device__ __forceinline__ void set_code(int k, u32 code) { fo::set_code<EPL>(out, k, code); }
+};
+
+// ref:2610-2676 _triton_quantize_kernel.  2 (4) bytes in and 1.06 out per element; two IEEE divisions (or one and an
+// IEEE root) per element would make it a matter of vector instructions (2.4 TB/s on bf16), so the two kinds of state
+// the optimizers hold go through the quick forms with verification, which give the same codes (fo_math.h).  Loading an
+// AdamW checkpoint of 2.2e8 weights (bf16, 24-bit masters; this kernel and Int8NarrowOp) takes 310 us, 6.4 TB/s, where
+// it took 912 with the IEEE form and torch's cast to int8 (1.3 TB/s).
+template <int XDT> struct QuantizeOp {
+    static constexpr int kEpl = DTypeInfo<XDT>::epl, kSpans = 2, kLutFloats = 4;
+    struct Raw { Pack<DTypeInfo<XDT>::bytes, kEpl> x; };
+    __device__ __forceinline__ static bool aligned(const fo_convert_job& j) { return aligned16(j.src, j.dst); }
+    template <int MODE> __device__ __forceinline__ static void load(const fo_convert_job& j, Where w, Raw& r) {
+        load_lane<DTypeInfo<XDT>::bytes, kEpl, MODE>(r.x, j.src, w, j.n);
+    }
+    __device__ __forceinline__ static void prepare(const fo_convert_job&, float*) {}
+    template <int MODE> __device__ __forceinline__ static void finish(const fo_convert_job& j, Where w, Raw& r, const float*) {
+        float v[kEpl];
+        float am = 0.0f;
+        Pack<1, kEpl> out;
+#pragma unroll
+        for (int k = 0; k < kEpl; ++k) v[k] = widen<XDT, kEpl>(r.x, k);
+        if (j.flags == (FO_CODEC_SIGNED | FO_CODEC_SOFTSIGN)) {
+#pragma unroll
+            for (int k = 0; k < kEpl; ++k) am = fmaxf(am, fabsf(v[k]));
+            am = fmaxf(group_max<kEpl>(am), 1e-12f);                            // ref:2657-2658
+            CodecLane<kEpl> lane{v, am, out};
+            HwWave<CodecLane<kEpl>> wave{lane};
+            codec_verified<kEpl, false>(wave);
+        } else if (j.flags == FO_CODEC_SQRT) {
+            // the root is monotone, so the largest root is the root of the largest value; negative values are NaN after
+            // the root and take no part in the maximum either way
+#pragma unroll
+            for (int k = 0; k < kEpl; ++k) am = fmaxf(am, v[k]);
+            am = fmaxf(sqrt_rn(group_max<kEpl>(am)), 1e-12f);
+            CodecLane<kEpl> lane{v, am, out};
+            HwWave<CodecLane<kEpl>> wave{lane};
+            codec_verified<kEpl, true>(wave);
+        } else {
+#pragma unroll
+            for (int k = 0; k < kEpl; ++k) {
+                if (j.flags & FO_CODEC_SQRT) v[k] = sqrt_rn(v[k]);              // ref:2650-2651
+                am = fmaxf(am, fabsf(v[k]));
+            }
+            am = fmaxf(group_max<kEpl>(am), 1e-12f);
+            const float out_max = (j.flags & FO_CODEC_SIGNED) ? 127.0f : 255.0f;
+            u32 q[kEpl];
+#pragma unroll
+            for (int k = 0; k < kEpl; ++k) {
+                const float nrm = div_rn(v[k], am);                             // ref:2661
+                const float t = (j.flags & FO_CODEC_SOFTSIGN) ? div_rn(2.0f * nrm, 1.0f + fabsf(nrm)) : nrm;   // ref:2664-2667
+                q[k] = (u32)(int)floorf(t * out_max + 0.5f);                    // ref:2670-2671
+            }
+            pack_codes<1, kEpl>(q, out);
+        }
+        store_lane<1, kEpl, MODE>(out, j.dst, w, j.n);
+        if ((MODE == kVector || w.first() < j.n) && (threadIdx.x & (32 / kEpl - 1)) == 0)                      // ref:2675-2676
+            store_scale(static_cast<uint16_t*>(j.dst2), w, f32_to_f16_bits(am));
+    }
+};
+
 // int8 codes as values of a 2-byte type (exact): the form in which a checkpoint holds 1-byte correction codes
 // (ref:900-927).  One byte in, two out.
 template <int DT> struct Int8WidenOp {
@@ -178,6 +222,25 @@ template <int DT> struct Int8WidenOp {
             narrow_pair<DT, 8>(o, k, ecc_to_float<1, 8>(r.codes, k), ecc_to_float<1, 8>(r.codes, k + 1), wa, wb);
         }
         store_lane<2, 8, MODE>(o, j.dst, w, j.n);
+    }
+};
+
+// The way back: values of a 2-byte type truncated to int8.
+template <int DT> struct Int8NarrowOp {
+    static constexpr int kEpl = 8, kSpans = 4, kLutFloats = 4;
+    struct Raw { Pack<2, 8> x; };
+    __device__ __forceinline__ static bool aligned(const fo_convert_job& j) { return aligned16(j.src, j.dst); }
+    template <int MODE> __device__ __forceinline__ static void load(const fo_convert_job& j, Where w, Raw& r) {
+        load_lane<2, 8, MODE>(r.x, j.src, w, j.n);
+    }
+    __device__ __forceinline__ static void prepare(const fo_convert_job&, float*) {}
+    template <int MODE> __device__ __forceinline__ static void finish(const fo_convert_job& j, Where w, Raw& r, const float*) {
+        u32 c[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) c[k] = (u32)(int)widen<DT, 8>(r.x, k);
+        Pack<1, 8> out;
+        pack_codes<1, 8>(c, out);
+        store_lane<1, 8, MODE>(out, j.dst, w, j.n);
     }
 };
 
@@ -223,12 +286,6 @@ __device__ __forceinline__ void ecc_split_lane(const float* x, const void* narro
         }                                                                                         \
     }
 
-template <int XDT>
-__global__ __launch_bounds__(kCodecThreads) void quantize_kernel(const void* x, void* codes, uint16_t* scales, int64_t n, CodecFlags f) {
-    const bool aligned = ((((uintptr_t)x) | ((uintptr_t)codes)) & 15u) == 0;
-    FO_SPAN_LOOP(n, DTypeInfo<XDT>::epl, aligned, (quantize_lane<XDT, true>(x, codes, scales, first, n, f)), (quantize_lane<XDT, false>(x, codes, scales, first, n, f)))
-}
-
 template <int DT, int ECCB>
 __global__ __launch_bounds__(kCodecThreads) void ecc_join_kernel(const void* narrow, const void* ecc, float* out, int64_t n) {
     const bool aligned = ((((uintptr_t)narrow) | ((uintptr_t)ecc) | ((uintptr_t)out)) & 15u) == 0;
@@ -250,6 +307,10 @@ using namespace fo_host;
 unsigned grid_for(int64_t n, int epl) {
     const int64_t spans = (n + 64 * epl - 1) / (64 * epl);
     return (unsigned)(spans < INT32_MAX ? spans : INT32_MAX);
+}
+
+int32_t codec_flags(int is_signed, int do_sqrt, int softsign) {
+    return (is_signed ? FO_CODEC_SIGNED : 0) | (do_sqrt ? FO_CODEC_SQRT : 0) | (softsign ? FO_CODEC_SOFTSIGN : 0);
 }
 
 // Enqueues the jobs, kJobsPerLaunch to a launch; the caller has checked their pointers.
@@ -308,16 +369,19 @@ int fo_quantize(const void* x, int x_dtype, void* codes, void* scales, int64_t n
     if (n == 0) return 0;  // ref:2485
     if (!x || !codes || !scales) return fail(FO_ERR_INVALID_ARGUMENT, "x, codes and scales must not be NULL");
     if (((uintptr_t)x & (x_dtype == FO_F32 ? 3 : 1)) || ((uintptr_t)scales & 1)) return fail(FO_ERR_INVALID_ARGUMENT, "x or scales not aligned to their element size");
-    if (compute_units() <= 0) return fail(FO_ERR_NO_DEVICE, "no HIP device");
-    const fo::CodecFlags f{is_signed ? 1 : 0, do_sqrt ? 1 : 0, softsign ? 1 : 0};
-    const dim3 grid(grid_for(n, x_dtype == FO_F32 ? 4 : 8)), block(fo::kCodecThreads);
+    const fo_convert_job job{x, nullptr, codes, scales, n, codec_flags(is_signed, do_sqrt, softsign), 0};
+    return fo_quantize_many(&job, 1, x_dtype, stream);
+}
+
+int fo_quantize_many(const fo_convert_job* jobs, int64_t n_jobs, int x_dtype, void* stream) {
+    if (x_dtype < FO_F32 || x_dtype > FO_F16) return fail(FO_ERR_INVALID_ARGUMENT, "unknown dtype %d", x_dtype);
+    if (int rc = validate_jobs(jobs, n_jobs, x_dtype == FO_F32 ? 4 : 2, 0, 1, 2)) return rc;
     hipStream_t s = (hipStream_t)stream;
     switch (x_dtype) {
-        case FO_F32: hipLaunchKernelGGL(fo::quantize_kernel<fo::DT_F32>, grid, block, 0, s, x, codes, (uint16_t*)scales, n, f); break;
-        case FO_BF16: hipLaunchKernelGGL(fo::quantize_kernel<fo::DT_BF16>, grid, block, 0, s, x, codes, (uint16_t*)scales, n, f); break;
-        default: hipLaunchKernelGGL(fo::quantize_kernel<fo::DT_F16>, grid, block, 0, s, x, codes, (uint16_t*)scales, n, f); break;
+        case FO_F32: return launch_jobs<fo::QuantizeOp<fo::DT_F32>>(jobs, n_jobs, s);
+        case FO_BF16: return launch_jobs<fo::QuantizeOp<fo::DT_BF16>>(jobs, n_jobs, s);
+        default: return launch_jobs<fo::QuantizeOp<fo::DT_F16>>(jobs, n_jobs, s);
     }
-    return check_hip(hipGetLastError(), "quantize kernel launch");
 }
 
 int fo_dequantize(const void* codes, const void* scales, float* out, int64_t n, int is_signed, int do_sqrt, int softsign,
@@ -326,8 +390,7 @@ int fo_dequantize(const void* codes, const void* scales, float* out, int64_t n, 
     if (n == 0) return 0;  // ref:2533
     if (!codes || !scales || !out) return fail(FO_ERR_INVALID_ARGUMENT, "codes, scales and out must not be NULL");
     if (((uintptr_t)out & 3) || ((uintptr_t)scales & 1)) return fail(FO_ERR_INVALID_ARGUMENT, "out or scales not aligned to their element size");
-    const int32_t flags = (is_signed ? FO_CODEC_SIGNED : 0) | (do_sqrt ? FO_CODEC_SQRT : 0) | (softsign ? FO_CODEC_SOFTSIGN : 0);
-    const fo_convert_job job{codes, scales, out, nullptr, n, flags, 0};
+    const fo_convert_job job{codes, scales, out, nullptr, n, codec_flags(is_signed, do_sqrt, softsign), 0};
     return fo_dequantize_many(&job, 1, FO_F32, stream);
 }
 
@@ -343,6 +406,13 @@ int fo_int8_widen_many(const fo_convert_job* jobs, int64_t n_jobs, int dtype, vo
     if (int rc = validate_jobs(jobs, n_jobs, 1, 0, 2, 0)) return rc;
     return dtype == FO_BF16 ? launch_jobs<fo::Int8WidenOp<fo::DT_BF16>>(jobs, n_jobs, (hipStream_t)stream)
                             : launch_jobs<fo::Int8WidenOp<fo::DT_F16>>(jobs, n_jobs, (hipStream_t)stream);
+}
+
+int fo_int8_narrow_many(const fo_convert_job* jobs, int64_t n_jobs, int dtype, void* stream) {
+    if (dtype != FO_BF16 && dtype != FO_F16) return fail(FO_ERR_INVALID_ARGUMENT, "dtype must be bf16 or fp16 (got %d)", dtype);
+    if (int rc = validate_jobs(jobs, n_jobs, 2, 0, 1, 0)) return rc;
+    return dtype == FO_BF16 ? launch_jobs<fo::Int8NarrowOp<fo::DT_BF16>>(jobs, n_jobs, (hipStream_t)stream)
+                            : launch_jobs<fo::Int8NarrowOp<fo::DT_F16>>(jobs, n_jobs, (hipStream_t)stream);
 }
 
 static int validate_ecc_args(const void* a, const void* b, const void* c, int narrow_dtype, int ecc_bytes, int64_t n) {

@@ -292,6 +292,20 @@ FO_FN u32 quantize_var_code_verified(float v, float av_quick, float av_exact) {
     return quick_value_is_safe(x, kQuickMarginVar) ? (u32)(int)x : quantize_var_code(sqrt_corrected(v), av_exact, hw::rcp(av_exact));
 }
 
+// The standalone codec's codes (fo_codec.hip), IEEE operation by operation as the reference writes them with plain
+// divisions and roots (ref:2650-2671): signed with softsign (first moments) and unsigned of the root (second moments).
+//   am: the group's largest |m|, resp. the correctly rounded root of its largest v, clamped at 1e-12.
+FO_FN u32 codec_mom_code(float m, float am) {
+    const float nm = m / am;
+    const float t = (2.0f * nm) / (1.0f + fabsf(nm));
+    return (u32)(int)floorf(t * 127.0f + 0.5f);
+}
+FO_FN u32 codec_var_code(float v, float am) { return (u32)(int)floorf(__builtin_sqrtf(v) / am * 255.0f + 0.5f); }
+// Quick forms of the same codes with the margins above: the IEEE forms stay closer to the real-number value than the
+// corrected quotients those margins allow for, and the second-moment form divides by the correctly rounded root here.
+// A group beyond kCodecLargest (infinities among them) would leave the quick forms' range: it takes the IEEE form.
+constexpr float kCodecLargest = 0x1p120f;
+
 // ------------------------------------------------------------------------------------------------
 // Adam / AdamW element update (ref:2296-2375)
 // ------------------------------------------------------------------------------------------------
@@ -524,6 +538,36 @@ template <int N, class Wave> FO_FN void requantize_both_verified(Wave& wave) {
                 wave.each([k](auto& L) FO_LANE_ATTR {
                     const u32 code = quantize_var_code(sqrt_corrected(L.v[k]), L.av, L.rav);
                     if (!quick_slack_is_safe(L.slack_v[k], kQuickMarginVar)) L.set_var_code(k, code);
+                });
+            }
+        }
+    }
+}
+
+// The standalone codec over a lane's N values of one kind (VAR: second moments).  Lane members:
+//   v[N], am            the values and what their group is divided by (codec_mom_code, codec_var_code)
+//   x[N], slack[N], least         scratch of the flow
+//   convert(x)          codes of all N values from their quick values
+//   set_code(k, c)      replaces the code of position k
+template <int N, bool VAR, class Wave> FO_FN void codec_verified(Wave& wave) {
+    constexpr float kMargin = VAR ? kQuickMarginVar : kQuickMarginMom;
+    wave.each([](auto& L) FO_LANE_ATTR {
+        const float ram255 = VAR ? hw::rcp(L.am) * 255.0f : 0.0f;
+        FO_UNROLL for (int k = 0; k < N; ++k) {
+            L.x[k] = VAR ? quantize_var_quick(hw::sqrt(L.v[k]), ram255) : quantize_mom_quick(L.v[k], L.am);
+            L.slack[k] = quick_value_slack(L.x[k]);
+        }
+        L.least = L.slack[0];
+        FO_UNROLL for (int k = 1; k < N; ++k) L.least = fminf(L.least, L.slack[k]);
+        L.convert(L.x);
+    });
+    if (wave.any([](const auto& L) FO_LANE_ATTR { return !(L.am < kCodecLargest) || !quick_slack_is_safe(L.least, kMargin); })) {
+        FO_UNROLL for (int k = 0; k < N; ++k) {
+            const auto redo = [k](const auto& L) FO_LANE_ATTR { return !(L.am < kCodecLargest) || !quick_slack_is_safe(L.slack[k], kMargin); };
+            if (wave.any(redo)) {
+                wave.each([k, &redo](auto& L) FO_LANE_ATTR {
+                    const u32 code = VAR ? codec_var_code(L.v[k], L.am) : codec_mom_code(L.v[k], L.am);
+                    if (redo(L)) L.set_code(k, code);
                 });
             }
         }

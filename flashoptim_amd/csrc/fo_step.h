@@ -89,21 +89,6 @@ __device__ __forceinline__ void write_master(const float (&p)[EPL], Pack<DTypeIn
     if constexpr (ECCB > 0) pack_codes<ECCB, EPL>(eb, eout);
 }
 
-// Replaces byte k of the lane's packed codes.
-template <int EPL> __device__ __forceinline__ void set_code(Pack<1, EPL>& out, int k, u32 code) {
-    const int sh = 8 * (k & 3);
-    u32& w = out.w[k >> 2];
-    w = (w & ~(0xffu << sh)) | ((code & 0xffu) << sh);
-}
-
-// The hardware wavefront as the verified flows of fo_math.h see it from one of its lanes: each() is one call on the
-// lane's own state, any() a ballot over the 64 lanes.
-template <class Lane> struct HwWave {
-    Lane& lane;
-    template <class F> __device__ __forceinline__ void each(F&& f) { f(lane); }
-    template <class P> __device__ __forceinline__ bool any(P&& p) { return __builtin_amdgcn_ballot_w64(p(lane)) != 0; }
-};
-
 // Lane state of requantize_mom_verified / requantize_var_verified for eight values per lane (2-byte parameters):
 // the codes are the two dwords that travel to memory; the conversion writes each byte in place (convert_pack8).
 struct MomLane8 {

@@ -55,6 +55,12 @@ def _check_group_size(group_size: int) -> None:
 # ------------------------------------------------------------------------------------------ group codec
 
 
+def _check_values(x: torch.Tensor) -> None:
+    _require_device(x, "quantize")
+    if x.dtype not in DTYPE_CODE:
+        raise ValueError(f"quantize expects fp32, bf16 or fp16 input, got {x.dtype}.")
+
+
 def quantize(
     x_float: torch.Tensor,
     out_int8: Optional[torch.Tensor] = None,
@@ -70,9 +76,7 @@ def quantize(
     scales are fp16 ``[ceil(N/32)]`` (ref:2476-2498).
     """
     _check_group_size(group_size)
-    _require_device(x_float, "quantize")
-    if x_float.dtype not in DTYPE_CODE:
-        raise ValueError(f"quantize expects fp32, bf16 or fp16 input, got {x_float.dtype}.")
+    _check_values(x_float)
     x = x_float if x_float.is_contiguous() else x_float.contiguous()
     n = x.numel()
     if out_int8 is None:
@@ -139,7 +143,9 @@ def dequantize(
 
 # --------------------------------------------------------------------------- conversions of many tensors
 
-_CODEC_SIGNED, _CODEC_SQRT, _CODEC_SOFTSIGN = 1, 2, 4  # fo_codec_flags
+
+def _codec_flags(signed: bool, sqrt: bool, softsign: bool) -> int:  # fo_codec_flags
+    return (1 if signed else 0) | (2 if sqrt else 0) | (4 if softsign else 0)
 
 
 class ConversionBatch:
@@ -166,8 +172,8 @@ class ConversionBatch:
         codes, scales = codes.contiguous(), scales.contiguous()
         out = torch.empty_like(codes, dtype=torch.bfloat16)
         if codes.numel() > 0:
-            flags = (_CODEC_SIGNED if signed else 0) | (_CODEC_SQRT if sqrt else 0) | (_CODEC_SOFTSIGN if softsign else 0)
-            self._add(("fo_dequantize_many", DTYPE_CODE[torch.bfloat16]), codes.device, codes, scales, out, None, flags)
+            self._add(("fo_dequantize_many", DTYPE_CODE[torch.bfloat16]), codes.device, codes, scales, out, None,
+                      _codec_flags(signed, sqrt, softsign))
         return out
 
     def widen_int8(self, values: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
@@ -178,6 +184,27 @@ class ConversionBatch:
         out = torch.empty_like(values, dtype=dtype)
         if values.numel() > 0:
             self._add(("fo_int8_widen_many", DTYPE_CODE[dtype]), values.device, values, None, out, None)
+        return out
+
+    def quantize(self, x: torch.Tensor, signed: bool, sqrt: bool, softsign: bool) -> tuple[torch.Tensor, torch.Tensor]:
+        """:func:`quantize` of one tensor."""
+        _check_values(x)
+        x = x.contiguous()
+        n = x.numel()
+        codes = torch.empty_like(x, dtype=torch.int8 if signed else torch.uint8)
+        scales = torch.empty((n + GROUP_SIZE - 1) // GROUP_SIZE, device=x.device, dtype=torch.float16)
+        if n > 0:
+            self._add(("fo_quantize_many", DTYPE_CODE[x.dtype]), x.device, x, None, codes, scales, _codec_flags(signed, sqrt, softsign))
+        return codes, scales
+
+    def narrow_to_int8(self, values: torch.Tensor) -> torch.Tensor:
+        """``values.to(torch.int8)`` of a bf16 or fp16 tensor."""
+        if (type(values) is not torch.Tensor or not values.is_cuda or not values.is_contiguous()
+                or values.dtype not in (torch.bfloat16, torch.float16)):
+            return values.to(dtype=torch.int8)
+        out = torch.empty_like(values, dtype=torch.int8)
+        if values.numel() > 0:
+            self._add(("fo_int8_narrow_many", DTYPE_CODE[values.dtype]), values.device, values, None, out, None)
         return out
 
     def launch(self) -> None:

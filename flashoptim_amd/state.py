@@ -106,7 +106,8 @@ class _MaybeQuantizedTensor:
         return self.scales if self.is_quantized() else self.kernel_tensor
 
     # -- value in / out ----------------------------------------------------------------------------
-    def set_data(self, data: torch.Tensor) -> None:
+    def set_data(self, data: torch.Tensor, batch: Optional[ConversionBatch] = None) -> None:
+        """Take over the values of `data`; with a `batch` a quantised state holds them once it is launched."""
         if self._try_quantize:
             if not data.is_cuda:
                 raise NotImplementedError(
@@ -114,7 +115,7 @@ class _MaybeQuantizedTensor:
                     f"{tuple(data.shape)}."
                 )
             self._data = None
-            self._quantized, self._scales = quantize(
+            self._quantized, self._scales = (quantize if batch is None else batch.quantize)(
                 data, signed=self._signed, sqrt=self._sqrt, softsign=self._softsign
             )
         else:
@@ -170,7 +171,7 @@ class _MaybeQuantizedTensor:
             own.launch()
         return {name: out}
 
-    def load_state_dict(self, d: dict[str, torch.Tensor], name: str) -> None:
+    def load_state_dict(self, d: dict[str, torch.Tensor], name: str, batch: Optional[ConversionBatch] = None) -> None:
         """Accepts the whole per-parameter state dict; only ``name`` and ``name::*`` are looked at (ref:191-210)."""
         mine = {k: v for k, v in d.items() if k == name or k.startswith(name + "::")}
         if name in mine:
@@ -178,7 +179,7 @@ class _MaybeQuantizedTensor:
                 raise ValueError(
                     f"If state dict specifies {name}, it must not specify other keys. Got {list(mine.keys())}"
                 )
-            self.set_data(mine[name])
+            self.set_data(mine[name], batch)
             return
         # torch.optim.Optimizer.load_state_dict has cast both tensors to the parameter dtype on the way in
         self._data = None
@@ -196,7 +197,8 @@ class _MaybeQuantizedTensor:
         sqrt: bool = False,
         softsign: bool = True,
         storage_dtype: torch.dtype = torch.float32,
+        batch: Optional[ConversionBatch] = None,
     ) -> "_MaybeQuantizedTensor":
         obj = cls(None, try_quantize=try_quantize, signed=signed, sqrt=sqrt, softsign=softsign, storage_dtype=storage_dtype)
-        obj.load_state_dict(d, name)
+        obj.load_state_dict(d, name, batch)
         return obj

@@ -200,7 +200,7 @@ int fo_ecc_split(const float *x, const void *narrow, int narrow_dtype, void *ecc
 
 /*
  * The conversions of a checkpoint over a list of tensors: what the reference runs as one kernel and one eager cast per
- * state of every parameter while it writes a state_dict (ref:159-167, 868-927).  `jobs` is a HOST array: the jobs travel as kernel arguments, 64 to a
+ * state of every parameter while it writes or reads a state_dict (ref:159-210, 797-927).  `jobs` is a HOST array: the jobs travel as kernel arguments, 64 to a
  * launch, so nothing is allocated, uploaded or synchronised, and the calls may be captured into a HIP graph.  Tensors
  * of different lengths share a launch; jobs of no elements are skipped.  All jobs of one call live on the
  * current device.
@@ -217,11 +217,14 @@ typedef struct fo_convert_job {
 
 enum fo_codec_flags { FO_CODEC_SIGNED = 1, FO_CODEC_SQRT = 2, FO_CODEC_SOFTSIGN = 4 };
 
+/* src = values (x_dtype), dst = codes, dst2 = scales */
+int fo_quantize_many(const fo_convert_job *jobs, int64_t n_jobs, int x_dtype, void *stream);
 /* src = codes, src2 = scales, dst = values: fp32, or bf16 rounded to nearest even from the fp32 value */
 int fo_dequantize_many(const fo_convert_job *jobs, int64_t n_jobs, int out_dtype, void *stream);
-/* int8 correction codes as values of the parameter's type, the form a checkpoint holds them in (ref:900-927):
- * src = int8, dst = `dtype` values (bf16 or fp16) */
+/* int8 correction codes as values of the parameter's type (bf16 or fp16), the form a checkpoint holds them in
+ * (ref:900-927): src = int8, dst = `dtype` values; and back, truncated towards zero: src = `dtype` values, dst = int8 */
 int fo_int8_widen_many(const fo_convert_job *jobs, int64_t n_jobs, int dtype, void *stream);
+int fo_int8_narrow_many(const fo_convert_job *jobs, int64_t n_jobs, int dtype, void *stream);
 
 #ifdef __cplusplus
 }

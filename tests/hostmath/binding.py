@@ -44,6 +44,8 @@ def lib() -> ctypes.CDLL:
         L.hm_flow_stats.restype = None
         L.hm_requantize_wave.argtypes = [vp] * 6
         L.hm_requantize_wave.restype = None
+        L.hm_codec_wave.argtypes = [vp, i32, vp, vp, vp]
+        L.hm_codec_wave.restype = None
         L.hm_code_over_255.argtypes = [vp]
         L.hm_code_over_255.restype = None
         L.hm_momentum_step.argtypes = [vp, vp, vp, vp, vp, i64, i32, i32, i32, f, f, f, f, i32, i32, i32]
@@ -125,6 +127,16 @@ def requantize_wave(m: torch.Tensor, v: torch.Tensor):
     out = [torch.empty(512, dtype=torch.uint8) for _ in range(4)]
     lib().hm_requantize_wave(_ptr(m.contiguous()), _ptr(v.contiguous()), *(t.data_ptr() for t in out))
     return out
+
+
+def codec_wave(x: torch.Tensor, var: bool):
+    """512 values (16 groups) through the standalone codec's verified flow.  Returns (its codes, the codes of the general
+    form, what each group is divided by)."""
+    assert x.numel() == 512 and x.dtype == torch.float32
+    quick, ieee = torch.empty(512, dtype=torch.uint8), torch.empty(512, dtype=torch.uint8)
+    am = torch.empty(16)
+    lib().hm_codec_wave(_ptr(x.contiguous()), int(var), quick.data_ptr(), ieee.data_ptr(), am.data_ptr())
+    return quick, ieee, am
 
 
 def code_over_255() -> torch.Tensor:

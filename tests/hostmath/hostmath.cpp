@@ -387,6 +387,34 @@ void hm_requantize_wave(const float* m, const float* v, uint8_t* qm, uint8_t* qv
         }
 }
 
+// One wavefront of the standalone codec: 512 values, lane l holding values 8l .. 8l+7, four lanes per group.  quick: codes
+// of the verified flow; ieee: of the general form, element by element; am: what each group is divided by.
+void hm_codec_wave(const float* x, int var, uint8_t* quick, uint8_t* ieee, float* am_out) {
+    struct Lane {
+        float v[8], am, x[8], slack[8], least;
+        u32 code[8];
+        void convert(const float (&q)[8]) { for (int k = 0; k < 8; ++k) code[k] = (u32)hw::floor_to_int(q[k]) & 0xffu; }
+        void set_code(int k, u32 c) { code[k] = c & 0xffu; ++g_stats.codes_replaced; }
+    };
+    static Lane ls[kLanes];
+    for (int g = 0; g < 16; ++g) {
+        float am = 0.0f;
+        for (int i = 0; i < 32; ++i) am = fmaxf(am, var ? x[32 * g + i] : fabsf(x[32 * g + i]));
+        am_out[g] = am = fmaxf(var ? sqrtf(am) : am, 1e-12f);
+        for (int l = 4 * g; l < 4 * g + 4; ++l) {
+            ls[l].am = am;
+            for (int k = 0; k < 8; ++k) ls[l].v[k] = x[8 * l + k];
+        }
+    }
+    SimWave<Lane> wave{ls};
+    if (var) codec_verified<8, true>(wave); else codec_verified<8, false>(wave);
+    for (int l = 0; l < kLanes; ++l)
+        for (int k = 0; k < 8; ++k) {
+            quick[8 * l + k] = (uint8_t)ls[l].code[k];
+            ieee[8 * l + k] = (uint8_t)(var ? codec_var_code(ls[l].v[k], ls[l].am) : codec_mom_code(ls[l].v[k], ls[l].am));
+        }
+}
+
 // Arguments as fo_adam_step (include/flashoptim_hip.h) without the stream; host pointers.
 // exact: <= 0 = the choice the kernels make for this variant (fo_adam_step), 1 = operation by operation on every
 // element (fo_adam_step_exact).  flagged (may be null): receives the number of elements whose folded update was

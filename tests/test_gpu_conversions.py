@@ -62,3 +62,42 @@ def test_widen_int8_over_a_list(dtype, offset):
     batch.launch()
     for values, got in cases:
         assert parity.bits_equal(got, values.to(dtype)), values.numel()
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("signed,sqrt,softsign", [(True, False, True), (False, True, False), (True, False, False), (False, True, True)])
+def test_quantize_over_a_list(signed, sqrt, softsign, dtype, offset):
+    """Continuous values, bf16 lattices, values on rounding boundaries and groups beyond the quick forms' range."""
+    from flashoptim_amd.kernels import ConversionBatch
+
+    g = torch.Generator().manual_seed(6)
+    batch, cases = ConversionBatch(), []
+    for n in _lengths(many=offset == 0):
+        x = torch.randn(n, generator=g) * 10.0 ** (n % 7 - 4)
+        if n % 3 == 0:
+            x = torch.randint(-127, 128, (n,), generator=g).float() / 127
+        x = (x if signed else x.abs()).to(dtype)
+        if n > 1024:
+            x[40], x[70], x[100] = torch.finfo(dtype).max, torch.finfo(dtype).tiny, 0.0
+            x[130:160] = 0.0
+        cases.append((x, batch.quantize(_at(x, offset), signed, sqrt, softsign)))
+    batch.launch()
+    for x, (codes, scales) in cases:
+        rc, rs = C.quantize(x, signed, sqrt, softsign)
+        assert torch.equal(codes.cpu(), rc), (x.numel(), "codes")
+        assert parity.bits_equal(scales, rs), (x.numel(), "scales")
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_narrow_to_int8_over_a_list(dtype, offset):
+    from flashoptim_amd.kernels import ConversionBatch
+
+    batch, cases = ConversionBatch(), []
+    for n in _lengths(many=offset == 0):
+        values = ((torch.arange(n) * 37 % 1021) / 4 - 127.75).clamp(-128, 127).to(dtype)
+        cases.append((values, batch.narrow_to_int8(_at(values, offset))))
+    batch.launch()
+    for values, got in cases:
+        assert torch.equal(got.cpu(), values.float().trunc().to(torch.int8)), values.numel()

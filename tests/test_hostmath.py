@@ -240,6 +240,38 @@ def test_verified_flows_repair_exactly_the_lane_and_position_that_failed(noise):
     assert H.flow_stats() == dict(waves=0, questions=10, yes=2, codes_replaced=2)
 
 
+@pytest.mark.parametrize("noise", [0, 7, 11])
+@pytest.mark.parametrize("var", [False, True])
+def test_codec_flow_gives_the_codes_of_the_general_form(var, noise):
+    """codec_verified over simulated wavefronts against the general form and the oracle's codec: continuous data, values on
+    rounding boundaries, lattices, bf16 values, and what leaves the quick forms' range (infinities, the type's largest
+    and smallest values, zeros, negative second moments, NaN)."""
+    from oracle import c_oracle as C
+
+    H.set_noise(noise)
+    g = torch.Generator().manual_seed(20 + noise)
+    normal = torch.randn(40, 512, generator=g)
+    waves = [w * 10.0 ** (i % 12 - 6) for i, w in enumerate(normal)]
+    waves += [w.to(torch.bfloat16).float() for w in normal[:8]]
+    waves += [torch.randint(-127, 128, (512,), generator=g).float() for _ in range(4)]
+    code = torch.arange(512).remainder(255) - 126.5
+    boundary = (code / 127) / (2 - (code / 127).abs()) if not var else ((code + 127) / 255) ** 2
+    waves += [boundary, boundary * 3e-3]
+    special = torch.tensor([0.0, -0.0, 1e-45, 1.1e-38, 1e-13, 1e30, 3.4e38, 2.0 ** 119, 2.0 ** 120, float("inf"), float("nan")])
+    for i in range(special.numel()):
+        w = normal[i].clone()
+        w[i * 7::64] = special[i]
+        waves += [w, w * 0 + special[i], torch.where(torch.arange(512) % 3 == 0, special[i], normal[i] * 1e-3)]
+    for i, w in enumerate(waves):
+        for x in ([w] if not var else [w, w.abs()]):
+            quick, ieee, am = H.codec_wave(x.float(), var)
+            assert torch.equal(quick, ieee), i
+            if torch.isfinite(x).all() and (not var or (x >= 0).all()):
+                codes, scales = C.quantize(x.float(), not var, var, not var)
+                assert torch.equal(quick, codes.view(torch.uint8)), i
+                assert parity.bits_equal(am.to(torch.float16), scales), i
+
+
 @pytest.mark.parametrize("noise", [0, 7])
 def test_update_repair_flow_redoes_the_one_flagged_element(noise):
     """adam_redo_flagged over simulated wavefronts: weights a thousand times larger than their updates except one, which

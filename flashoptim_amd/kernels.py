@@ -159,6 +159,8 @@ class ConversionBatch:
     def __init__(self) -> None:
         self._jobs: dict = {}  # (entry point, *its leading arguments, device) -> flat list of fo_convert_job words
         self._keepalive: list = []  # inputs must outlive the launch
+        self._import_sources: set = set()  # storages that pending imports read
+        self._import_targets: set = set()  # storages and addresses that pending imports write
 
     def _add(self, entry: tuple, device: torch.device, src: torch.Tensor, src2, dst: torch.Tensor, dst2, flags: int = 0) -> None:
         ptr = _native.ptr
@@ -207,6 +209,26 @@ class ConversionBatch:
             self._add(("fo_int8_narrow_many", DTYPE_CODE[values.dtype]), values.device, values, None, out, None)
         return out
 
+    def import_fp32(self, x: torch.Tensor, narrow: torch.Tensor, error_bits: torch.Tensor) -> Optional[torch.Tensor]:
+        """``narrow.copy_(x)`` and the new correction term ``compute_ecc_bits(x, narrow, ...)`` of `error_bits`' width in
+        one pass; None (and nothing done) where the tensors are not laid out for it."""
+        if (not type(x) is type(narrow) is torch.Tensor or x.dtype != torch.float32 or x.shape != narrow.shape
+                or not x.is_contiguous() or not narrow.is_contiguous() or not narrow.is_cuda or x.device != narrow.device
+                or narrow.dtype not in (torch.bfloat16, torch.float16) or error_bits.element_size() not in (1, 2)):
+            return None
+        source, target = x.untyped_storage().data_ptr(), narrow.untyped_storage().data_ptr()
+        if source == target:
+            return None
+        if source in self._import_targets or target in self._import_sources or ("at", narrow.data_ptr()) in self._import_targets:
+            self.launch()  # tensors that share memory keep the order of the calls; jobs of one launch have none
+        self._import_sources.add(source)
+        self._import_targets.update((target, ("at", narrow.data_ptr())))
+        width = error_bits.element_size()
+        out = torch.empty(narrow.shape, dtype=torch.int8 if width == 1 else torch.int16, device=narrow.device)
+        if narrow.numel() > 0:
+            self._add(("fo_ecc_narrow_many", DTYPE_CODE[narrow.dtype], width), narrow.device, x, None, narrow, out)
+        return out
+
     def launch(self) -> None:
         """Enqueue everything collected so far on the current stream of each device."""
         jobs, self._jobs = self._jobs, {}
@@ -216,6 +238,13 @@ class ConversionBatch:
                 rc = getattr(_native.lib(), name)(table, len(words) // 6, *args, _native.current_stream_ptr(device))
             _native.check(rc, name)
         self._keepalive.clear()
+        self._import_sources.clear()
+        self._import_targets.clear()
+
+    def launch_if_reading(self, t: torch.Tensor) -> None:
+        """``launch()`` if a pending import reads the memory of `t`, which is about to be written."""
+        if self._import_sources and t.untyped_storage().data_ptr() in self._import_sources:
+            self.launch()
 
 
 # ------------------------------------------------------------------------------------------------- ECC

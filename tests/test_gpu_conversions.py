@@ -101,3 +101,61 @@ def test_narrow_to_int8_over_a_list(dtype, offset):
     batch.launch()
     for values, got in cases:
         assert torch.equal(got.cpu(), values.float().trunc().to(torch.int8)), values.numel()
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ecc_dtype", [torch.int8, torch.int16])
+def test_import_fp32_over_a_list(ecc_dtype, dtype, offset):
+    """Against the cast, the copy and the split it stands for, over magnitudes down to subnormals, infinities and NaN."""
+    from flashoptim_amd.kernels import ConversionBatch, compute_ecc_bits
+
+    g = torch.Generator().manual_seed(8)
+    special = torch.tensor([0.0, -0.0, 1e-40, 3e38, float("inf"), -float("inf"), float("nan"), 1 + 2.0 ** -8, -(1 + 2.0 ** -9)])
+    batch, cases = ConversionBatch(), []
+    for n in _lengths(many=offset == 0):
+        x = torch.exp(torch.empty(n).uniform_(-90, 12, generator=g)) * torch.where(torch.rand(n, generator=g) < 0.5, -1.0, 1.0)
+        x[: min(n, 9)] = special[: min(n, 9)]
+        x = _at(x, offset)
+        narrow = _at(torch.zeros(n, dtype=dtype), offset)
+        cases.append((x, narrow, batch.import_fp32(x, narrow, torch.empty(n, dtype=ecc_dtype, device=DEV))))
+    batch.launch()
+    for x, narrow, ecc in cases:
+        want = x.to(dtype)
+        assert torch.equal(narrow.view(torch.int16), want.view(torch.int16)), x.numel()
+        assert ecc.dtype == ecc_dtype
+        assert torch.equal(ecc, compute_ecc_bits(x, want, master_bytewidth=2 + ecc.element_size())), x.numel()
+
+
+def test_import_fp32_declines_what_it_would_write_wrongly():
+    from flashoptim_amd.kernels import ConversionBatch
+
+    x, e = torch.zeros(8, 6, device=DEV), torch.zeros(8, 6, device=DEV, dtype=torch.int8)
+    p = torch.zeros(8, 6, device=DEV, dtype=torch.bfloat16)
+    declined = [(x.t(), p, e), (x, p.t(), e), (x[:1], p, e), (x.view(48), p, e), (x.cpu(), p, e), (x, x, e), (x.half(), p, e)]
+    assert all(ConversionBatch().import_fp32(*args) is None for args in declined)
+
+
+def test_imports_that_share_memory_keep_their_order():
+    """Two parameters over one memory (the last import wins), and a value that lives in a parameter imported later."""
+    import flashoptim_amd as fo
+
+    class Holder(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            n = 5000
+            self.a = torch.nn.Parameter(torch.zeros(n, device=DEV, dtype=torch.bfloat16))
+            self.b = torch.nn.Parameter(torch.zeros(0, device=DEV, dtype=torch.bfloat16))
+            self.b.data = self.a.data
+            self.c = torch.nn.Parameter(torch.full((n,), 3.0, device=DEV))
+
+    m = Holder()
+    opt = fo.FlashAdamW(m.parameters(), lr=1e-3)
+    for p in m.parameters():
+        p.grad = torch.zeros_like(p)
+    opt.step()
+    n = m.a.numel()
+    opt.set_fp32_model_state_dict(m, {"a": m.c.data, "b": torch.full((n,), 2.0, device=DEV), "c": torch.full((n,), 9.0, device=DEV)})
+    assert (m.a == 2.0).all() and (m.b == 2.0).all() and (m.c == 9.0).all()
+    opt.set_fp32_model_state_dict(m, {"b": m.c.data, "c": torch.full((n,), 4.0, device=DEV)})
+    assert (m.b == 9.0).all() and (m.c == 4.0).all()

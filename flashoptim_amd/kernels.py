@@ -216,6 +216,10 @@ class ConversionBatch:
                 or not x.is_contiguous() or not narrow.is_contiguous() or not narrow.is_cuda or x.device != narrow.device
                 or narrow.dtype not in (torch.bfloat16, torch.float16) or error_bits.element_size() not in (1, 2)):
             return None
+        width = error_bits.element_size()
+        out = torch.empty(narrow.shape, dtype=torch.int8 if width == 1 else torch.int16, device=narrow.device)
+        if narrow.numel() == 0:
+            return out
         source, target = x.untyped_storage().data_ptr(), narrow.untyped_storage().data_ptr()
         if source == target:
             return None
@@ -223,10 +227,7 @@ class ConversionBatch:
             self.launch()  # tensors that share memory keep the order of the calls; jobs of one launch have none
         self._import_sources.add(source)
         self._import_targets.update((target, ("at", narrow.data_ptr())))
-        width = error_bits.element_size()
-        out = torch.empty(narrow.shape, dtype=torch.int8 if width == 1 else torch.int16, device=narrow.device)
-        if narrow.numel() > 0:
-            self._add(("fo_ecc_narrow_many", DTYPE_CODE[narrow.dtype], width), narrow.device, x, None, narrow, out)
+        self._add(("fo_ecc_narrow_many", DTYPE_CODE[narrow.dtype], width), narrow.device, x, None, narrow, out)
         return out
 
     def launch(self) -> None:

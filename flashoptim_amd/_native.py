@@ -80,6 +80,7 @@ SIGNATURES = {
     "fo_dequantize_many": (_i32, [_vp, _i64, _i32, _vp]),
     "fo_int8_widen_many": (_i32, [_vp, _i64, _i32, _vp]),
     "fo_int8_narrow_many": (_i32, [_vp, _i64, _i32, _vp]),
+    "fo_ecc_join_many": (_i32, [_vp, _i64, _i32, _i32, _vp]),
     "fo_ecc_narrow_many": (_i32, [_vp, _i64, _i32, _i32, _vp]),
     "fo_quantize_many": (_i32, [_vp, _i64, _i32, _vp]),
     "fo_ecc_join": (_i32, [_vp, _i32, _vp, _i32, _vp, _i64, _vp]),

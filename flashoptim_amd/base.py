@@ -23,7 +23,7 @@ import torch
 import torch.nn as nn
 
 from . import _hostscan, kernels
-from .kernels import compute_ecc_bits, reconstruct_fp32_param
+from .kernels import compute_ecc_bits
 from .launcher import BucketPlan, StepTensors
 from .state import QuantizedTensorSpec, _MaybeQuantizedTensor
 
@@ -723,11 +723,19 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
     def get_fp32_model_state_dict(self, model: nn.Module) -> dict[str, torch.Tensor]:
         """The model's state dict in fp32, with ECC-corrected master weights where available (ref:1035-1084)."""
         module = cast(nn.Module, model.module if hasattr(model, "module") else model)
-        out = {k: v.detach().float() for k, v in module.state_dict().items()}
+        batch = kernels.ConversionBatch()  # every parameter with a correction term in one launch
+        masters = {}
         for name, param in module.named_parameters():
             ecc = self.state.get(param, {}).get("error_bits")
             if ecc is not None:
-                out[name] = reconstruct_fp32_param(self._get_local_tensor(param.detach()), ecc)
+                masters[name] = batch.reconstruct_fp32(self._get_local_tensor(param.detach()), ecc)
+        out = {}
+        for k, v in module.state_dict().items():
+            # no cast of a narrow weight whose master takes its place
+            replaced = k in masters and type(v) is torch.Tensor and v.dtype in (torch.bfloat16, torch.float16)
+            out[k] = masters[k] if replaced else v.detach().float()
+        out.update(masters)
+        batch.launch()
         return out
 
     def set_fp32_model_state_dict(self, model: nn.Module, fp32_state_dict: dict[str, torch.Tensor]) -> None:

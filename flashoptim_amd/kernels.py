@@ -228,6 +228,18 @@ class ConversionBatch:
         self._import_sources.add(source)
         self._import_targets.update((target, ("at", narrow.data_ptr())))
         self._add(("fo_ecc_narrow_many", DTYPE_CODE[narrow.dtype], width), narrow.device, x, None, narrow, out)
+<<<<<<< Updated upstream
+=======
+        return out
+
+    def reconstruct_fp32(self, param: torch.Tensor, error_bits: torch.Tensor) -> torch.Tensor:
+        """:func:`reconstruct_fp32_param` of one parameter."""
+        _check_join(param, error_bits)
+        out = torch.empty(param.shape, dtype=torch.float32, device=param.device)
+        if param.numel() > 0:
+            self._add(("fo_ecc_join_many", DTYPE_CODE[param.dtype], error_bits.element_size()), param.device,
+                      param.contiguous(), error_bits.contiguous(), out, None)
+>>>>>>> Stashed changes
         return out
 
     def launch(self) -> None:
@@ -251,8 +263,7 @@ class ConversionBatch:
 # ------------------------------------------------------------------------------------------------- ECC
 
 
-def reconstruct_fp32_param(param: torch.Tensor, error_bits: torch.Tensor) -> torch.Tensor:
-    """fp32 master weights from a bf16/fp16 parameter and its int8/int16 correction term (ref:2835-2892)."""
+def _check_join(param: torch.Tensor, error_bits: torch.Tensor) -> None:
     if param.dtype == torch.float32:
         raise ValueError(
             "param is already fp32; ECC reconstruction is only meaningful for narrow dtypes (bf16, fp16). "
@@ -266,17 +277,13 @@ def reconstruct_fp32_param(param: torch.Tensor, error_bits: torch.Tensor) -> tor
     if error_bits.numel() != param.numel():
         raise ValueError("error_bits must have as many elements as param")
     _require_same_device(param, error_bits, "error_bits")
-    out = torch.empty(param.shape, dtype=torch.float32, device=param.device)
-    n = param.numel()
-    if n > 0:
-        narrow = param.contiguous()
-        ecc = error_bits.contiguous()
-        with _native.device_guard(param.device):
-            rc = _native.lib().fo_ecc_join(
-                narrow.data_ptr(), DTYPE_CODE[param.dtype], ecc.data_ptr(), ecc.element_size(), out.data_ptr(), n,
-                _native.current_stream_ptr(param.device),
-            )
-        _native.check(rc, "fo_ecc_join")
+
+
+def reconstruct_fp32_param(param: torch.Tensor, error_bits: torch.Tensor) -> torch.Tensor:
+    """fp32 master weights from a bf16/fp16 parameter and its int8/int16 correction term (ref:2835-2892)."""
+    batch = ConversionBatch()
+    out = batch.reconstruct_fp32(param, error_bits)
+    batch.launch()
     return out
 
 

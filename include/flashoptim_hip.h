@@ -226,7 +226,9 @@ int fo_dequantize_many(const fo_convert_job *jobs, int64_t n_jobs, int out_dtype
 int fo_int8_widen_many(const fo_convert_job *jobs, int64_t n_jobs, int dtype, void *stream);
 int fo_int8_narrow_many(const fo_convert_job *jobs, int64_t n_jobs, int dtype, void *stream);
 
-/* fp32 master weights into the parameters (ref:1086-1147): src = fp32, dst = narrow_dtype values rounded to nearest even,
+/* fp32 master weights out of the parameters (ref:1035-1084): src = narrow_dtype values, src2 = their ecc, dst = fp32 */
+int fo_ecc_join_many(const fo_convert_job *jobs, int64_t n_jobs, int narrow_dtype, int ecc_bytes, void *stream);
+/* and into them (ref:1086-1147): src = fp32, dst = narrow_dtype values rounded to nearest even,
  * dst2 = their ecc, as fo_ecc_split gives it for src and dst */
 int fo_ecc_narrow_many(const fo_convert_job *jobs, int64_t n_jobs, int narrow_dtype, int ecc_bytes, void *stream);
 

@@ -127,6 +127,54 @@ def test_import_fp32_over_a_list(ecc_dtype, dtype, offset):
         assert torch.equal(ecc, compute_ecc_bits(x, want, master_bytewidth=2 + ecc.element_size())), x.numel()
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ecc_dtype", [torch.int8, torch.int16])
+def test_export_fp32_over_a_list(ecc_dtype, dtype, offset):
+    from flashoptim_amd.kernels import ConversionBatch
+
+    g = torch.Generator().manual_seed(9)
+    special = torch.tensor([0.0, -0.0, 1e-40, 6e-8, float("inf"), -float("inf")])
+    top = torch.iinfo(ecc_dtype).max
+    batch, cases = ConversionBatch(), []
+    for n in _lengths(many=offset == 0):
+        w = torch.randn(n, generator=g) * 10.0 ** (n % 9 - 5)
+        w[: min(n, 6)] = special[: min(n, 6)]
+        w = w.to(dtype)
+        ecc = torch.randint(-top, top + 1, (n,), generator=g).to(ecc_dtype)
+        cases.append((w, ecc, batch.reconstruct_fp32(_at(w, offset), _at(ecc, offset))))
+    batch.launch()
+    for w, ecc, got in cases:
+        want = C.ecc_join(w, ecc)
+        assert torch.equal(got.cpu().nan_to_num(7.0), want.nan_to_num(7.0)), w.numel()
+
+
+def test_fp32_export_of_a_module_with_buffers_tied_and_fp32_weights():
+    """Keys, their order and every value as the per-tensor sequence gives them: parameters with a correction term as their
+    masters (a tied one under its first name only), everything else cast."""
+    import flashoptim_amd as fo
+
+    m = torch.nn.Module()
+    m.a = torch.nn.Parameter(torch.randn(33, 70, device=DEV).to(torch.bfloat16))
+    m.b = torch.nn.Parameter(torch.randn(1000, device=DEV))
+    m.c = torch.nn.Parameter(torch.randn(40, 25, device=DEV).to(torch.bfloat16).t())  # not contiguous: never stepped
+    m.register_buffer("buf", torch.arange(5, device=DEV))
+    m.tied = m.a
+    m.d = torch.nn.Parameter(torch.zeros(0, device=DEV, dtype=torch.bfloat16))
+    opt = fo.FlashAdamW(m.parameters(), lr=1e-3)
+    for p in (m.a, m.b, m.d):
+        p.grad = torch.randn_like(p)
+    opt.step()
+    opt.state[m.c]["error_bits"] = torch.randint(-127, 128, m.c.shape, device=DEV, dtype=torch.int8)
+    want = {k: v.detach().float() for k, v in m.state_dict().items()}
+    for k, p in (("a", m.a), ("c", m.c), ("d", m.d)):
+        want[k] = C.ecc_join(p.detach().contiguous().cpu(), opt.state[p]["error_bits"].contiguous().cpu()).view(p.shape).to(DEV)
+    got = opt.get_fp32_model_state_dict(m)
+    assert list(got) == list(want)
+    for k, v in want.items():
+        assert got[k].dtype == torch.float32 and got[k].shape == v.shape and torch.equal(got[k], v), k
+
+
 def test_import_fp32_declines_what_it_would_write_wrongly():
     from flashoptim_amd.kernels import ConversionBatch
 

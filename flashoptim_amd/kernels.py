@@ -228,8 +228,6 @@ class ConversionBatch:
         self._import_sources.add(source)
         self._import_targets.update((target, ("at", narrow.data_ptr())))
         self._add(("fo_ecc_narrow_many", DTYPE_CODE[narrow.dtype], width), narrow.device, x, None, narrow, out)
-<<<<<<< Updated upstream
-=======
         return out
 
     def reconstruct_fp32(self, param: torch.Tensor, error_bits: torch.Tensor) -> torch.Tensor:
@@ -239,7 +237,6 @@ class ConversionBatch:
         if param.numel() > 0:
             self._add(("fo_ecc_join_many", DTYPE_CODE[param.dtype], error_bits.element_size()), param.device,
                       param.contiguous(), error_bits.contiguous(), out, None)
->>>>>>> Stashed changes
         return out
 
     def launch(self) -> None:

@@ -8,6 +8,7 @@ from typing import Any, Literal, Optional
 
 import torch
 
+from . import _hostscan
 from .base import FlashOptimizer
 from .state import QuantizedTensorSpec
 
@@ -93,6 +94,9 @@ class FlashAdam(FlashOptimizer):
         return "exp_avg", "exp_avg_sq"
 
     def _advance_step(self, param_state: dict[str, Any]) -> Optional[int]:
+        step = None if _hostscan.advance is None else _hostscan.advance(param_state["step"])
+        if step is not None:
+            return int(step)
         param_state["step"] += 1
         return int(param_state["step"].item())
 

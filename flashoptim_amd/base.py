@@ -319,9 +319,9 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
         errors: Optional[torch.Tensor],
         param_state: dict[str, Any],
         hparams: dict[str, Any],
-    ) -> tuple[LaunchKey, StepTensors]:
+    ) -> tuple[str, bool, dict[str, Any], StepTensors]:
         """Host-side part of one parameter's step: advance counters, fold the hyper-parameters into the kernel
-        scalars and name the tensors."""
+        scalars and name the tensors.  Returns kernel kind, whether the states are quantised, scalars, tensors."""
         if errors is not None and errors.dtype not in (torch.int8, torch.int16):
             raise ValueError("Errors needs to be int8 or int16")
         kind = self._kernel_kind(hparams)
@@ -329,8 +329,6 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
         mom_name, var_name = self._moment_names(kind)
         mom = param_state[mom_name] if mom_name else None
         var = param_state[var_name] if var_name else None
-        key = LaunchKey(kind, param.dtype, 0 if errors is None else errors.element_size(),
-                        mom.is_quantized() if mom is not None else False, tuple(sorted(scalars.items())), param.device)
         tensors = StepTensors(
             param=param, grad=grad, ecc=errors,
             mom=None if mom is None else mom.kernel_tensor,
@@ -338,9 +336,19 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
             var=None if var is None else var.kernel_tensor,
             var_scales=None if var is None else var.kernel_scales_or_self,
         )
-        return key, tensors
+        return kind, mom.is_quantized() if mom is not None else False, scalars, tensors
 
     def _plan_param(self, p: torch.Tensor, group: dict[str, Any]) -> Optional[tuple[LaunchKey, StepTensors]]:
+        """A parameter's step up to the launch, with the key that says which tensors may share one."""
+        plan = self._prepare_param(p, group)
+        if plan is None:
+            return None
+        kind, quantized, scalars, t = plan
+        key = LaunchKey(kind, t.param.dtype, 0 if t.ecc is None else t.ecc.element_size(), quantized,
+                        tuple(sorted(scalars.items())), t.param.device)
+        return key, t
+
+    def _prepare_param(self, p: torch.Tensor, group: dict[str, Any]) -> Optional[tuple[str, bool, dict[str, Any], StepTensors]]:
         """Everything ``step_param`` does short of launching (ref:699-759)."""
         if id(p) not in self._state_ready or not self.state.get(p):
             self._ensure_state_initialized(p, hparams=group)
@@ -372,16 +380,15 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
         return self._plan_step(p_local, grad_local, param_state.get("error_bits"), param_state, group)
 
     @staticmethod
-    def _launch_single(key: LaunchKey, t: StepTensors) -> None:
-        kw = dict(key.scalars)
-        if key.kind == "adam":
+    def _launch_single(kind: str, quantized: bool, scalars: dict[str, Any], t: StepTensors) -> None:
+        if kind == "adam":
             kernels._fused_adam_step(t.mom, t.mom_scales, t.var, t.var_scales, t.param, t.grad, t.ecc,
-                                     quantize_optim_states=key.quantized, **kw)
-        elif key.kind == "momentum":
+                                     quantize_optim_states=quantized, **scalars)
+        elif kind == "momentum":
             kernels._fused_momentum_step(t.mom, t.mom_scales, t.param, t.grad, t.ecc,
-                                         quantize_optim_states=key.quantized, **kw)
+                                         quantize_optim_states=quantized, **scalars)
         else:
-            kernels._sgd_plain_step(t.param, t.grad, t.ecc, **kw)
+            kernels._sgd_plain_step(t.param, t.grad, t.ecc, **scalars)
 
     @torch.no_grad()
     def step_param(self, p: torch.Tensor, group: Optional[dict[str, Any]] = None) -> None:
@@ -395,7 +402,7 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
             group = self._find_group(p)
         self._refuse_graph_capture()
         self._plan_epoch += 1  # counters move outside step(): cached bucket state is stale
-        plan = self._plan_param(p, group)
+        plan = self._prepare_param(p, group)
         if plan is not None:
             self._launch_single(*plan)
 
@@ -438,7 +445,7 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
                 plan.launch(**scalars)
             else:
                 for t in tensors:
-                    self._launch_single(key, t)
+                    self._launch_single(key.kind, key.quantized, scalars, t)
             step_pool, step_views = None, None
             if "step" in scalars:
                 # the per-parameter CPU `step` scalars become 0-dim views into one tensor, so that the cached path
@@ -475,13 +482,18 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
                 # the counters are live state the caller may have rewritten (a warm restart zeroes them): take the
                 # step number from them, and leave counters that no longer agree to the per-parameter path.  A
                 # counter OBJECT that was replaced (state[p]["step"] = tensor(0.)) no longer aliases the pool.
-                state = self.state
-                if [id(state[p].get("step")) for p in b.params] != b.step_view_ids:
-                    return False
-                lo, hi = torch.aminmax(b.step_pool)
-                lo = lo.item()
-                if lo != hi.item():
-                    return False
+                if _hostscan.counters is not None:
+                    lo = _hostscan.counters(self.state, b.params, b.step_views, b.step_pool)
+                    if lo is None:
+                        return False
+                else:
+                    state = self.state
+                    if [id(state[p].get("step")) for p in b.params] != b.step_view_ids:
+                        return False
+                    lo, hi = torch.aminmax(b.step_pool)
+                    lo = lo.item()
+                    if lo != hi.item():
+                        return False
                 b.step_value = int(lo)
             if b.plan is None:  # single-tensor bucket: launched from the live tensors below
                 for p in b.params:
@@ -514,16 +526,16 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
             plan.set_grad_ptr(i, ptr)
         for b in cache.buckets:
             if b.step_pool is not None:
-                b.step_pool.add_(1)
+                if _hostscan.advance is None or _hostscan.advance(b.step_pool) is None:
+                    b.step_pool.add_(1)
                 b.step_value += 1
             scalars = self._kernel_scalars(group, b.step_value)
             if b.plan is not None:
                 b.plan.launch(**scalars)
             else:
-                key = LaunchKey(b.kind, b.dtype, b.ecc_bytes, b.quantized, tuple(sorted(scalars.items())))
                 for p, t in zip(b.params, b.tensors):
                     t.grad = p.grad
-                    self._launch_single(key, t)
+                    self._launch_single(b.kind, b.quantized, scalars, t)
                     t.grad = None
         return True
 

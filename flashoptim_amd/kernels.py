@@ -14,7 +14,7 @@ from typing import Optional
 
 import torch
 
-from . import _native
+from . import _hostscan, _native
 from ._native import DTYPE_CODE
 
 GROUP_SIZE = 32
@@ -364,6 +364,27 @@ def _check_moment(param: torch.Tensor, values: torch.Tensor, scales: Optional[to
     _require_same_device(param, scales, f"{name} scales")
 
 
+def _step_args(param: torch.Tensor, grad: torch.Tensor, errors: Optional[torch.Tensor], mom: Optional[torch.Tensor],
+               mom_scales: Optional[torch.Tensor], var: Optional[torch.Tensor], var_scales: Optional[torch.Tensor],
+               quantized: bool) -> tuple:
+    """The checked arguments of a single-tensor step: addresses of mom, mom_scales, var, var_scales, param, grad, errors,
+    then elements, dtype code, ECC bytes.  The checks run in C++ where the helper is built (0.4 instead of 4 us); what
+    it does not vouch for comes here, and the exceptions are raised here."""
+    if _hostscan.step_args is not None:
+        args = _hostscan.step_args(param, grad, errors, mom, mom_scales, var, var_scales, quantized)
+        if args is not None:
+            return args
+    _check_step_tensors(param, grad, errors)
+    if mom is not None:
+        _check_moment(param, mom, mom_scales, quantized, True, "mom" if var is not None else "momentum")
+    if var is not None:
+        _check_moment(param, var, var_scales, quantized, False, "var")
+    ecc_bytes = _ecc_bytes(errors)
+    ptr = _native.ptr
+    return (ptr(mom), ptr(mom_scales) if quantized else None, ptr(var), ptr(var_scales) if quantized else None,
+            param.data_ptr(), grad.data_ptr(), ptr(errors), param.numel(), DTYPE_CODE[param.dtype], ecc_bytes)
+
+
 def _fused_adam_step(
     mom: torch.Tensor,
     mom_scales_f16: torch.Tensor,
@@ -394,19 +415,11 @@ def _fused_adam_step(
     n = param.numel()
     if n == 0:
         return
-    _check_step_tensors(param, grad, errors)
-    _check_moment(param, mom, mom_scales_f16, quantize_optim_states, True, "mom")
-    _check_moment(param, var, var_scales_f16, quantize_optim_states, False, "var")
-    ecc_bytes = _ecc_bytes(errors)
+    args = _step_args(param, grad, errors, mom, mom_scales_f16, var, var_scales_f16, quantize_optim_states)
     with _native.device_guard(param.device):
         entry = _native.lib().fo_adam_step_exact if exact_update else _native.lib().fo_adam_step
-        rc = entry(
-            mom.data_ptr(), mom_scales_f16.data_ptr() if quantize_optim_states else None,
-            var.data_ptr(), var_scales_f16.data_ptr() if quantize_optim_states else None,
-            param.data_ptr(), grad.data_ptr(), _native.ptr(errors), n, DTYPE_CODE[param.dtype], ecc_bytes,
-            int(quantize_optim_states), lr, beta1, beta2, eps, weight_decay, int(decoupled), int(step),
-            _native.current_stream_ptr(param.device),
-        )
+        rc = entry(*args, int(quantize_optim_states), lr, beta1, beta2, eps, weight_decay, int(decoupled), int(step),
+                   _native.current_stream_ptr(param.device))
     _native.check(rc, "fo_adam_step")
 
 
@@ -431,15 +444,11 @@ def _fused_momentum_step(
     n = param.numel()
     if n == 0:
         return
-    _check_step_tensors(param, grad, errors)
-    _check_moment(param, momentum, scales_f16, quantize_optim_states, True, "momentum")
-    ecc_bytes = _ecc_bytes(errors)
+    mom_ptr, scales_ptr, _, _, *args = _step_args(param, grad, errors, momentum, scales_f16, None, None, quantize_optim_states)
     with _native.device_guard(param.device):
         rc = _native.lib().fo_momentum_step(
-            momentum.data_ptr(), scales_f16.data_ptr() if quantize_optim_states else None, param.data_ptr(),
-            grad.data_ptr(), _native.ptr(errors), n, DTYPE_CODE[param.dtype], ecc_bytes,
-            int(quantize_optim_states), lr, mom_coef, update_coef, weight_decay, int(decoupled), int(nesterov),
-            int(do_lion), _native.current_stream_ptr(param.device),
+            mom_ptr, scales_ptr, *args, int(quantize_optim_states), lr, mom_coef, update_coef, weight_decay,
+            int(decoupled), int(nesterov), int(do_lion), _native.current_stream_ptr(param.device),
         )
     _native.check(rc, "fo_momentum_step")
 
@@ -457,12 +466,9 @@ def _sgd_plain_step(
     n = param.numel()
     if n == 0:
         return
-    _check_step_tensors(param, grad, errors)
+    args = _step_args(param, grad, errors, None, None, None, None, False)
     with _native.device_guard(param.device):
-        rc = _native.lib().fo_sgd_plain_step(
-            param.data_ptr(), grad.data_ptr(), _native.ptr(errors), n, DTYPE_CODE[param.dtype], _ecc_bytes(errors),
-            lr, weight_decay, int(decoupled), _native.current_stream_ptr(param.device),
-        )
+        rc = _native.lib().fo_sgd_plain_step(*args[4:], lr, weight_decay, int(decoupled), _native.current_stream_ptr(param.device))
     _native.check(rc, "fo_sgd_plain_step")
 
 

@@ -138,6 +138,9 @@ class BucketPlan:
         self.chunks_dev = host.to(self.device)
         nbytes = self.n_tensors * ctypes.sizeof(FoTensorDesc)
         self.descs_dev = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        # what every launch of the plan starts its argument list with
+        self._head = (self.descs_dev.data_ptr(), self.n_tensors, self.chunks_dev.data_ptr(), self.n_chunks,
+                      DTYPE_CODE[dtype], self.ecc_bytes, int(self.quantized))
         # two pinned staging buffers for the life of the plan, used in turn; `_staged[i]` marks the last copy out of
         # buffer i
         self._staging = [torch.empty(nbytes, dtype=torch.uint8).pin_memory() for _ in range(2)]
@@ -182,8 +185,7 @@ class BucketPlan:
             if self._dirty:
                 self._upload()
             lib = _native.lib()
-            head = (self.descs_dev.data_ptr(), self.n_tensors, self.chunks_dev.data_ptr(), self.n_chunks,
-                    DTYPE_CODE[self.dtype], self.ecc_bytes, int(self.quantized))
+            head = self._head
             stream = _native.current_stream_ptr(self.device)
             if self.kind == "adam":
                 entry = lib.fo_multi_adam_step_exact if scalars.get("exact_update") else lib.fo_multi_adam_step

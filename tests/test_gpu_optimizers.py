@@ -1356,3 +1356,74 @@ def test_a_tensor_stepped_as_shards_equals_the_whole_tensor(factory, kwargs):
         assert float((pa - pb).abs().max()) <= 2.0 * kwargs["lr"] * step, f"ragged split, step {step}"
         assert float((pa - pb).abs().mean()) <= 0.05 * kwargs["lr"] * step, f"ragged split, step {step}"
     assert not parity.bits_equal(whole[-1][names[0]], ragged[-1][names[0]])          # the groups behind the cut are other groups
+
+
+# ------------------------------------------------------------------------- arguments of single-tensor launches
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("quantized", [True, False])
+def test_step_arguments_checked_in_cpp_equal_the_python_checks(dtype, quantized, monkeypatch):
+    """The same addresses and sizes from both, and every tensor that the Python checks refuse is declined in C++."""
+    from flashoptim_amd import _hostscan
+    from flashoptim_amd import kernels as K
+
+    n = 100
+    z = lambda dt, m=n, **kw: torch.zeros(m, dtype=dt, device=DEV, **kw)  # noqa: E731
+    mom, var = (z(torch.int8), z(torch.uint8)) if quantized else (z(dtype), z(dtype))
+    scales = (z(torch.float16, 4), z(torch.float16, 5)) if quantized else (mom, var)
+    good = dict(param=torch.nn.Parameter(z(dtype)), grad=z(dtype), errors=None if dtype == torch.float32 else z(torch.int8),
+                mom=mom, mom_scales=scales[0], var=var, var_scales=scales[1], quantized=quantized)
+    forms = [good, {**good, "var": None, "var_scales": None}, {**good, "mom": None, "mom_scales": None, "var": None, "var_scales": None}]
+    if dtype != torch.float32:
+        forms += [{**good, "errors": z(torch.int16)}, {**good, "errors": None}]
+    bad = [{"grad": z(dtype, n + 1)}, {"grad": z(dtype).cpu()}, {"grad": z(dtype, 2 * n)[::2]}, {"grad": z(torch.float64)},
+           {"errors": z(torch.int32)}, {"errors": z(torch.int8, n - 1)}, {"errors": z(torch.int8, 2 * n)[::2]},
+           {"mom": z(torch.float64)}, {"mom": z(mom.dtype, n - 1)}, {"var": z(torch.int64)}, {"var": z(var.dtype).cpu()},
+           {"param": torch.nn.Parameter(z(torch.float64))}]
+    if quantized:
+        bad += [{"mom_scales": z(torch.float16, 3)}, {"mom_scales": None}, {"var_scales": z(torch.float32, 4)},
+                {"var_scales": z(torch.float16, 8)[::2]}, {"mom": z(torch.uint8)}]
+    native = [_hostscan.step_args(*f.values()) for f in forms]
+    assert all(_hostscan.step_args(*{**good, **b}.values()) is None for b in bad)
+    monkeypatch.setattr(_hostscan, "step_args", None)
+    for f, got in zip(forms, native):
+        want = K._step_args(*f.values())
+        assert [x or 0 for x in got] == [x or 0 for x in want]
+    for b in bad:
+        with pytest.raises((ValueError, RuntimeError, NotImplementedError)):
+            K._step_args(*{**good, **b}.values())
+
+
+@pytest.mark.parametrize("name", ["FlashAdamW", "FlashLion", "FlashSGD"])
+def test_host_helper_and_python_step_alike(name, monkeypatch):
+    """step() over a list, step() over one tensor and step_param() with the C++ helper and without it."""
+    from flashoptim_amd import _hostscan
+
+    fo = _fo()
+
+    def run():
+        out = []
+        for shapes in ([70, 4097, 1], [513]):
+            params = _make_params(shapes, torch.bfloat16, 31)
+            kw = dict(momentum=0.9) if name == "FlashSGD" else {}
+            opt = getattr(fo, name)(params, lr=1e-2, **kw)
+            for it in range(6):
+                _set_grads(params, 7 + it)
+                if it == 3:
+                    for p in params:
+                        opt.step_param(p)
+                else:
+                    opt.step()
+                if it == 4 and name == "FlashAdamW":
+                    assert all(float(opt.state[p]["step"]) == 5.0 for p in params)
+                    opt.state[params[0]]["step"].fill_(1.0)
+            out += [p.detach().clone() for p in params]
+        return out
+
+    native = run()
+    for f in ("scan", "same_objects", "counters", "advance", "step_args"):
+        assert getattr(_hostscan, f) is not None
+        monkeypatch.setattr(_hostscan, f, None)
+    for a, b in zip(native, run()):
+        assert torch.equal(a, b)

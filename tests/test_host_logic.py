@@ -444,3 +444,70 @@ def test_hostscan_module_validates_a_launch_table_like_the_python_walk():
     assert _hostscan.same_objects(params, list(params)) and not _hostscan.same_objects(params, params[:-1])
     assert not _hostscan.same_objects(params, params[1:] + params[:1])
     del keep
+
+
+def test_hostscan_counters_agree_with_the_python_walk():
+    import collections
+
+    from flashoptim_amd import _hostscan
+
+    class Odd(torch.nn.Parameter):  # a key whose hash is not its address
+        def __hash__(self):
+            return 7
+
+    def python_walk(state, params, views, pool):
+        if [id(state.get(p, {}).get("step")) for p in params] != list(map(id, views)):
+            return None
+        lo, hi = torch.aminmax(pool)
+        return lo.item() if lo.item() == hi.item() else None
+
+    for dict_type in (dict, lambda: collections.defaultdict(dict)):
+        params = [torch.nn.Parameter(torch.zeros(3)) for _ in range(5)] + [Odd(torch.zeros(2))]
+        pool = torch.full((6,), 4.0)
+        views = [pool[i] for i in range(6)]
+        state = dict_type()
+        for p, v in zip(params, views):
+            state[p] = {"step": v}
+        walk = lambda: (_hostscan.counters(state, params, views, pool), python_walk(state, params, views, pool))  # noqa: E731
+        assert walk() == (4.0, 4.0)
+        for i, value in ((3, 5.0), (0, float("nan"))):
+            pool[i] = value
+            assert walk() == (None, None)
+            pool[i] = 4.0
+        state[params[2]]["step"] = torch.tensor(4.0)       # a replaced counter object
+        assert walk() == (None, None)
+        state[params[2]] = {"step": views[2]}              # a replaced entry with the right counter
+        assert walk() == (4.0, 4.0)
+        del state[params[4]]
+        assert walk() == (None, None)
+        assert params[4] not in state                      # looking does not create it
+        state[params[4]] = {}
+        assert walk() == (None, None)
+    assert _hostscan.counters(state, params, views, torch.zeros(6, dtype=torch.float64)) is None
+    assert _hostscan.counters(state, [], [], torch.zeros(0)) is None
+
+
+def test_hostscan_advance_moves_cpu_fp32_counters_only():
+    from flashoptim_amd import _hostscan
+
+    pool = torch.tensor([1.0, 1.0, 1.0])
+    version = pool._version
+    assert _hostscan.advance(pool) == 2.0 and pool.tolist() == [2.0] * 3 and pool._version > version
+    assert _hostscan.advance(pool[1]) == 3.0 and pool.tolist() == [2.0, 3.0, 2.0]
+    with torch.inference_mode():
+        frozen = torch.zeros(2)
+    for other in (torch.zeros(2, dtype=torch.float64), torch.zeros(2, dtype=torch.int64), torch.zeros(0), torch.zeros(4)[::2], 3,
+                  torch.zeros(2, requires_grad=True), torch.empty(2, device="meta"), frozen):
+        before = other.tolist() if isinstance(other, torch.Tensor) and other.device.type == "cpu" else None
+        assert _hostscan.advance(other) is None
+        assert before is None or other.tolist() == before
+
+
+def test_hostscan_step_args_declines_what_is_not_on_a_gpu():
+    from flashoptim_amd import _hostscan
+
+    p = torch.zeros(64)
+    assert _hostscan.step_args(p, p.clone(), None, p.clone(), None, None, None, False) is None
+    assert _hostscan.step_args(p, None, None, None, None, None, None, False) is None
+    with pytest.raises(TypeError):
+        _hostscan.step_args(p)

@@ -52,6 +52,21 @@ static_assert(sizeof(JobBatch) <= 3584, "a batch must fit the kernel argument se
 
 // Op: kEpl elements per lane and span, kSpans neighbouring spans of 64 * kEpl elements per workgroup; a Raw holds
 // what a lane has loaded for one span; all loads of a workgroup are issued before the first span is finished.
+// kSpans is each Op's best over five sets of 2^27 elements in turn (more than the caches hold), bf16 where the type is
+// free (TB/s of the bytes in and out):
+//     spans per workgroup         1      2      3      4      6      8
+//     fp32 masters out          6.01   6.54   6.33   6.42   6.14   6.34
+//     fp32 masters in           6.09   6.66   6.38   6.43   6.11   6.08
+//     dequantise to bf16        4.81   6.51   6.15   6.35   6.00   6.18
+//     dequantise to fp32        3.99   5.54   5.92   6.30   5.90   6.15
+//     quantise, first moments   4.20   6.08   6.07   6.28   5.92   6.02
+//     quantise, second moments  4.02   5.49   5.56   5.91   5.77   5.70
+//     quantise fp32             4.55   5.80   6.04   6.49   6.38   6.18
+//     int8 to bf16              5.28   6.56   6.16   6.24   6.13   6.17
+//     bf16 to int8              5.66   6.67   6.35   6.43   6.27   6.15
+// One span leaves what a workgroup costs to start (its place in the list, the table in LDS, the spread of its loads) over
+// too few bytes, many spans widen the window of addresses in flight; odd counts start workgroups at odd KiB.  A cap on the
+// resident workgroups gains nothing on top.
 template <class Op> struct ConvertShape {
     static constexpr int64_t kSpan = 64 * Op::kEpl;
     static constexpr int64_t kBlock = kSpan * Op::kSpans;
@@ -89,12 +104,11 @@ template <int DT> __device__ __forceinline__ float one_nan(float x) { return (DT
 
 // ref:2541-2607 _triton_dequantize_kernel, with the cast to the output type that follows it in a checkpoint (ref:167).
 // Bound by memory: 1.06 bytes in and 4 (fp32) or 2 (bf16) out per element.  kSpans: the 1 KiB table that a workgroup
-// copies to LDS serves 1024 (fp32) or 2048 (bf16) elements; with one span per workgroup fp32 reached 4.7 instead of
-// 5.6 TB/s, reading the table through the vector cache instead 3.5.  An AdamW checkpoint of 2.2e8 weights (bf16, 24-bit
-// masters; this kernel and Int8WidenOp) takes 315 us, 6.3 TB/s, where fp32 values, their casts and torch's int8 cast
+// copies to LDS serves 1024 elements; reading the table through the vector cache instead is slower by a third.  An AdamW checkpoint of 2.2e8 weights (bf16, 24-bit
+// masters; this kernel and Int8WidenOp) takes 307 us, 6.5 TB/s, where fp32 values, their casts and torch's int8 cast
 // (1.3 TB/s) took 1456.
 template <int ODT> struct DequantizeOp {
-    static constexpr int kEpl = DTypeInfo<ODT>::epl, kSpans = 4, kLutFloats = 256;
+    static constexpr int kEpl = DTypeInfo<ODT>::epl, kSpans = ODT == DT_F32 ? 4 : 2, kLutFloats = 256;
     struct Raw { Pack<1, kEpl> codes; uint16_t scale; };
     __device__ __forceinline__ static bool aligned(const fo_convert_job& j) { return aligned16(j.src, j.dst); }
     template <int MODE> __device__ __forceinline__ static void load(const fo_convert_job& j, Where w, Raw& r) {
@@ -149,10 +163,10 @@ template <int EPL> struct CodecLane {
 // ref:2610-2676 _triton_quantize_kernel.  2 (4) bytes in and 1.06 out per element; two IEEE divisions (or one and an
 // IEEE root) per element would make it a matter of vector instructions (2.4 TB/s on bf16), so the two kinds of state
 // the optimizers hold go through the quick forms with verification, which give the same codes (fo_math.h).  Loading an
-// AdamW checkpoint of 2.2e8 weights (bf16, 24-bit masters; this kernel and Int8NarrowOp) takes 310 us, 6.4 TB/s, where
+// AdamW checkpoint of 2.2e8 weights (bf16, 24-bit masters; this kernel and Int8NarrowOp) takes 301 us, 6.6 TB/s, where
 // it took 912 with the IEEE form and torch's cast to int8 (1.3 TB/s).
 template <int XDT> struct QuantizeOp {
-    static constexpr int kEpl = DTypeInfo<XDT>::epl, kSpans = 2, kLutFloats = 4;
+    static constexpr int kEpl = DTypeInfo<XDT>::epl, kSpans = 4, kLutFloats = 4;
     struct Raw { Pack<DTypeInfo<XDT>::bytes, kEpl> x; };
     __device__ __forceinline__ static bool aligned(const fo_convert_job& j) { return aligned16(j.src, j.dst); }
     template <int MODE> __device__ __forceinline__ static void load(const fo_convert_job& j, Where w, Raw& r) {
@@ -207,7 +221,7 @@ template <int XDT> struct QuantizeOp {
 // int8 codes as values of a 2-byte type (exact): the form in which a checkpoint holds 1-byte correction codes
 // (ref:900-927).  One byte in, two out.
 template <int DT> struct Int8WidenOp {
-    static constexpr int kEpl = 8, kSpans = 4, kLutFloats = 4;
+    static constexpr int kEpl = 8, kSpans = 2, kLutFloats = 4;
     struct Raw { Pack<1, 8> codes; };
     __device__ __forceinline__ static bool aligned(const fo_convert_job& j) { return aligned16(j.src, j.dst); }
     template <int MODE> __device__ __forceinline__ static void load(const fo_convert_job& j, Where w, Raw& r) {
@@ -227,7 +241,7 @@ template <int DT> struct Int8WidenOp {
 
 // The way back: values of a 2-byte type truncated to int8.
 template <int DT> struct Int8NarrowOp {
-    static constexpr int kEpl = 8, kSpans = 4, kLutFloats = 4;
+    static constexpr int kEpl = 8, kSpans = 2, kLutFloats = 4;
     struct Raw { Pack<2, 8> x; };
     __device__ __forceinline__ static bool aligned(const fo_convert_job& j) { return aligned16(j.src, j.dst); }
     template <int MODE> __device__ __forceinline__ static void load(const fo_convert_job& j, Where w, Raw& r) {
@@ -246,9 +260,9 @@ template <int DT> struct Int8NarrowOp {
 
 // Import of fp32 master weights: the cast to the parameter's type and the correction codes of what it rounded off
 // (ref:2806-2832 _compute_ecc_bits_kernel) in one pass, 4 bytes in and 3 or 4 out per element:
-// 2.2e8 weights (bf16, 24-bit masters) take 241 us, 6.3 TB/s, where a cast, a copy and the split took 594.
+// 2.2e8 weights (bf16, 24-bit masters) take 230 us, 6.6 TB/s, where a cast, a copy and the split took 594.
 template <int DT, int ECCB> struct EccNarrowOp {
-    static constexpr int kEpl = 4, kSpans = 4, kLutFloats = 4;
+    static constexpr int kEpl = 4, kSpans = 2, kLutFloats = 4;
     struct Raw { Pack<4, 4> x; };
     __device__ __forceinline__ static bool aligned(const fo_convert_job& j) { return aligned16(j.src, j.dst) && aligned16(j.dst2, nullptr); }
     template <int MODE> __device__ __forceinline__ static void load(const fo_convert_job& j, Where w, Raw& r) {
@@ -274,10 +288,10 @@ template <int DT, int ECCB> struct EccNarrowOp {
 };
 
 // ref:2779-2803 _reconstruct_fp32_kernel, the way out again: narrow value and correction code in (3 or 4 bytes), the fp32
-// master out.  Bound by memory: 2.2e8 weights (bf16, 24-bit masters) take 241 us, 6.3 TB/s; the export of a model took
+// master out.  Bound by memory: 2.2e8 weights (bf16, 24-bit masters) take 232 us, 6.6 TB/s; the export of a model took
 // 483 as long as it also cast every narrow weight and joined tensor by tensor.
 template <int DT, int ECCB> struct EccJoinOp {
-    static constexpr int kEpl = 4, kSpans = 4, kLutFloats = 4;
+    static constexpr int kEpl = 4, kSpans = 2, kLutFloats = 4;
     struct Raw { Pack<2, 4> narrow; Pack<ECCB, 4> ecc; };
     __device__ __forceinline__ static bool aligned(const fo_convert_job& j) { return aligned16(j.src, j.dst) && aligned16(j.src2, nullptr); }
     template <int MODE> __device__ __forceinline__ static void load(const fo_convert_job& j, Where w, Raw& r) {

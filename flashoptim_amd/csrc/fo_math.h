@@ -185,13 +185,15 @@ template <int DT, int ECCB, bool CLAMP> FO_FN u32 ecc_split_bits(float p, float 
         const float s = as_f32(0x7ffe0000u - pow2_of_exponent_bits<DT>(widened));
         return as_u32(hw::fma(err, s, 1536.0f));
     } else {
-        const int nls = (DTypeInfo<DT>::mant + 1 + 127) - (int)(pow2_of_exponent_bits<DT>(widened) >> 23);
-        float en = hw::ldexp(err, nls);
-        if constexpr (CLAMP) en = hw::med3(en, -1.0f, 1.0f);
+        // err * 2^(1 - E), exact (0x7f800000 minus the pattern of 2^E is the pattern of 2^(1 - E), a normal number for every
+        // exponent field 1..254), then the rest of the scaling with MAX in one rounded product
+        constexpr float kRest = (float)(1 << DTypeInfo<DT>::mant);
+        float en = err * as_f32(0x7f800000u - pow2_of_exponent_bits<DT>(widened));
+        if constexpr (CLAMP) en = hw::med3(en, -1.0f / kRest, 1.0f / kRest);
         if constexpr (DT == DT_BF16 && ECCB == 1) {
-            return as_u32(hw::fma(en, EccInfo<ECCB>::max_val, kMagic));
+            return as_u32(hw::fma(en, EccInfo<ECCB>::max_val * kRest, kMagic));
         } else {
-            const float sc = en * EccInfo<ECCB>::max_val;
+            const float sc = en * (EccInfo<ECCB>::max_val * kRest);
             return (u32)(int)(sc + __builtin_copysignf(0.5f, sc));
         }
     }
@@ -255,6 +257,12 @@ FO_FN u32 quantize_var_code(float r, float av, float rav) { return (u32)(int)qua
 // 2^-24 relative, each approximate instruction at most an ulp; in code units, with |x| <= 128 resp. 256):
 //     first moment   exact 3.8e-5, quick 3.8e-5   ->  they can differ by 7.6e-5   ->  margin 2^-13 = 1.2e-4
 //     second moment  exact 7.6e-5, quick 1.2e-4   ->  they can differ by 2.0e-4   ->  margin 2^-12 = 2.4e-4
+// The operation-by-operation Adam update has a root at hand, of v / bc2 (a quotient, correctly rounded, and a corrected
+// root: 1.5u with u = 2^-24).  The quick form takes it in place of hw::sqrt(v), whose instruction costs four issue slots,
+// and av / sqrt(bc2) (two roundings more, 2u) in place of av: 9.5u instead of 8u on a value up to 256, 1.45e-4 for the
+// quick form, 2.2e-4 together.  v / bc2 must not overflow for that, so a group whose largest root reaches kQuickLargestVar
+// takes the exact form (bc2, one minus an fp32 power, is zero or at least 2^-24; where it is zero every root is a NaN,
+// which fails the test too).
 // so when the quick value lies farther than the margin from every integer, floor() of it IS the exact form's code.
 // Precondition: am + |m| and av stay below 2^126 (beyond that the reciprocal instruction returns a subnormal, flushed
 // to zero).  The group scale is stored as fp16 and overflows at 65504, forty orders of magnitude earlier, so a state
@@ -269,6 +277,7 @@ FO_FN u32 quantize_var_code(float r, float av, float rav) { return (u32)(int)qua
 // kernels on 2-byte parameters; the other kernels evaluate the exact forms only.
 constexpr float kQuickMarginMom = 0x1p-13f;
 constexpr float kQuickMarginVar = 0x1p-12f;
+constexpr float kQuickLargestVar = 0x1p48f;
 // Quick pre-floor values (margin included).  rav255 = 255 * rcp(av), av = hw::sqrt of the group's largest v.
 FO_FN float quantize_mom_quick(float m, float am) {
     const float t = m * hw::rcp(am + fabsf(m));  // = nm / (1 + |nm|), nm = m / am
@@ -324,6 +333,7 @@ struct AdamHyper {
     int folded_ok;
     // operation-by-operation form (EXACT): the reference's own sequence with correctly rounded quotients
     float lr, eps, bc1, rcp_bc1, bc2, rcp_bc2;  // rcp_*: correctly rounded reciprocals, formed on the host
+    float rcp_sqrt_bc2;                         // 1 / sqrt(bc2)
 };
 
 // Host side: the constants of one launch from the reference's kernel arguments (ref:2264-2270).
@@ -337,6 +347,7 @@ inline AdamHyper make_adam_hyper(float lr, float beta1, float beta2, float eps, 
     h.bc2 = 1.0f - (float)std::pow((double)beta2, (double)step);
     h.rcp_bc1 = (float)(1.0 / (double)h.bc1);
     h.rcp_bc2 = (float)(1.0 / (double)h.bc2);
+    h.rcp_sqrt_bc2 = (float)(1.0 / std::sqrt((double)h.bc2));
     h.lr = lr; h.eps = eps;
     const double bc1 = (double)h.bc1, bc2 = (double)h.bc2;
     if (lr != 0.0f) {
@@ -385,11 +396,13 @@ FO_FN void adam_moments_plain(float g, float mo, float vo, const AdamHyper& h, f
 }
 
 // p -= lr * (m/bc1) / (sqrt(v/bc2) + eps), operation by operation (ref:2368-2375): every quotient and the root
-// correctly rounded.  p: the weight after the decoupled decay, if any.
-FO_FN float adam_apply_exact(float p, float mn, float vn, const AdamHyper& h) {
+// correctly rounded.  p: the weight after the decoupled decay, if any.  `root` receives sqrt(v/bc2), from which the
+// requantiser's quick form of the second moment starts (kQuickMarginVar).
+FO_FN float adam_apply_exact(float p, float mn, float vn, const AdamHyper& h, float& root) {
     const float cm = div_corrected(mn, h.bc1, h.rcp_bc1);
     const float cv = div_corrected(vn, h.bc2, h.rcp_bc2);
-    const float den = sqrt_corrected(cv) + h.eps;
+    root = sqrt_corrected(cv);
+    const float den = root + h.eps;
     float rd = hw::rcp(den);
     rd = hw::fma(hw::fma(-den, rd, 1.0f), rd, rd);  // reciprocal refined to well below an ulp
     return p - div_corrected(h.lr * cm, den, rd);
@@ -479,7 +492,11 @@ template <int N, class Wave> FO_FN void requantize_mom_verified(Wave& wave) {
 //   av_quick, av        hw::sqrt and sqrt_corrected of the group's largest v (clamped at 1e-12)
 //   x[N], slack[N], least, rav    scratch of the flow
 //   convert_var(x), set_var_code(k, c)
-template <int N, class Wave> FO_FN void requantize_var_verified(Wave& wave) {
+// SCALED: r are the roots of v / bc2, and av_quick the quick root of the largest v over the root of bc2.
+template <bool SCALED, class Lane> FO_FN bool quick_var_is_safe(const Lane& L, float slack) {
+    return (!SCALED || L.av < kQuickLargestVar) && quick_slack_is_safe(slack, kQuickMarginVar);
+}
+template <int N, bool SCALED = false, class Wave> FO_FN void requantize_var_verified(Wave& wave) {
     wave.each([](auto& L) FO_LANE_ATTR {
         const float rav255 = hw::rcp(L.av_quick) * 255.0f;
         FO_UNROLL for (int k = 0; k < N; ++k) {
@@ -490,13 +507,13 @@ template <int N, class Wave> FO_FN void requantize_var_verified(Wave& wave) {
         FO_UNROLL for (int k = 1; k < N; ++k) L.least = fminf(L.least, L.slack[k]);
         L.convert_var(L.x);
     });
-    if (wave.any([](const auto& L) FO_LANE_ATTR { return !quick_slack_is_safe(L.least, kQuickMarginVar); })) {
+    if (wave.any([](const auto& L) FO_LANE_ATTR { return !quick_var_is_safe<SCALED>(L, L.least); })) {
         wave.each([](auto& L) FO_LANE_ATTR { L.rav = hw::rcp(L.av); });
         FO_UNROLL for (int k = 0; k < N; ++k) {
-            if (wave.any([k](const auto& L) FO_LANE_ATTR { return !quick_slack_is_safe(L.slack[k], kQuickMarginVar); })) {
+            if (wave.any([k](const auto& L) FO_LANE_ATTR { return !quick_var_is_safe<SCALED>(L, L.slack[k]); })) {
                 wave.each([k](auto& L) FO_LANE_ATTR {
                     const u32 code = quantize_var_code(sqrt_corrected(L.v[k]), L.av, L.rav);
-                    if (!quick_slack_is_safe(L.slack[k], kQuickMarginVar)) L.set_var_code(k, code);
+                    if (!quick_var_is_safe<SCALED>(L, L.slack[k])) L.set_var_code(k, code);
                 });
             }
         }
@@ -506,7 +523,7 @@ template <int N, class Wave> FO_FN void requantize_var_verified(Wave& wave) {
 // Both moments of a lane that holds N values of each (fp32 parameters, N = 4): one conversion, one repair branch.
 // Lane members: those of the two flows above with the scratch doubled (xm, xv, slack_m, slack_v, least_m, least_v)
 // and convert_both(xm, xv).
-template <int N, class Wave> FO_FN void requantize_both_verified(Wave& wave) {
+template <int N, bool SCALED = false, class Wave> FO_FN void requantize_both_verified(Wave& wave) {
     wave.each([](auto& L) FO_LANE_ATTR {
         const float rav255 = hw::rcp(L.av_quick) * 255.0f;
         FO_UNROLL for (int k = 0; k < N; ++k) {
@@ -524,7 +541,7 @@ template <int N, class Wave> FO_FN void requantize_both_verified(Wave& wave) {
         L.convert_both(L.xm, L.xv);
     });
     if (wave.any([](const auto& L) FO_LANE_ATTR {
-            return !quick_slack_is_safe(L.least_m, kQuickMarginMom) || !quick_slack_is_safe(L.least_v, kQuickMarginVar);
+            return !quick_slack_is_safe(L.least_m, kQuickMarginMom) || !quick_var_is_safe<SCALED>(L, L.least_v);
         })) {
         wave.each([](auto& L) FO_LANE_ATTR { L.ram = hw::rcp(L.am); L.rav = hw::rcp(L.av); });
         FO_UNROLL for (int k = 0; k < N; ++k) {
@@ -534,10 +551,10 @@ template <int N, class Wave> FO_FN void requantize_both_verified(Wave& wave) {
                     if (!quick_slack_is_safe(L.slack_m[k], kQuickMarginMom)) L.set_mom_code(k, code);
                 });
             }
-            if (wave.any([k](const auto& L) FO_LANE_ATTR { return !quick_slack_is_safe(L.slack_v[k], kQuickMarginVar); })) {
+            if (wave.any([k](const auto& L) FO_LANE_ATTR { return !quick_var_is_safe<SCALED>(L, L.slack_v[k]); })) {
                 wave.each([k](auto& L) FO_LANE_ATTR {
                     const u32 code = quantize_var_code(sqrt_corrected(L.v[k]), L.av, L.rav);
-                    if (!quick_slack_is_safe(L.slack_v[k], kQuickMarginVar)) L.set_var_code(k, code);
+                    if (!quick_var_is_safe<SCALED>(L, L.slack_v[k])) L.set_var_code(k, code);
                 });
             }
         }
@@ -591,7 +608,8 @@ template <int N, bool DECOUPLED, class Wave> FO_FN void adam_redo_flagged(Wave& 
                 wave.each([k, &h](auto& L) FO_LANE_ATTR {
                     float pk = L.old_master(k);
                     if (DECOUPLED) pk = pk * h.one_m_wd;                                // ref:2363-2364
-                    const float pe = adam_apply_exact(pk, L.m[k], L.v[k], h);           // ref:2368-2375
+                    float root;
+                    const float pe = adam_apply_exact(pk, L.m[k], L.v[k], h, root);     // ref:2368-2375
                     if (adam_folded_is_flagged(L.slack[k])) L.p[k] = pe;
                 });
             }

@@ -142,23 +142,25 @@ __device__ __forceinline__ void quantize_mom_quick_verified(const float (&m)[EPL
     HwWave<MomLane8> wave{lane};
     requantize_mom_verified<8>(wave);
 }
-// r: hw::sqrt of the lane's second moments v; av_quick / av_exact: hw::sqrt and sqrt_corrected of the group's largest v.
-template <int EPL>
+// r: hw::sqrt of the lane's second moments v; av_quick / av_exact: hw::sqrt and sqrt_corrected of the group's largest v
+// (SCALED: r and av_quick scaled as requantize_var_verified says).
+template <int EPL, bool SCALED>
 __device__ __forceinline__ void quantize_var_quick_verified(const float (&v)[EPL], const float (&r)[EPL], float av_quick,
                                                             float av_exact, Pack<1, EPL>& out) {
     static_assert(EPL == 8, "two dwords of codes per lane");
     VarLane8 lane{v, r, av_quick, av_exact, out};
     HwWave<VarLane8> wave{lane};
-    requantize_var_verified<8>(wave);
+    requantize_var_verified<8, SCALED>(wave);
 }
 // Four elements per lane (fp32 parameters), both states through the quick forms with verification: one conversion
 // block, one repair branch.
+template <bool SCALED>
 __device__ __forceinline__ void quantize_mom_var_quick_verified(const float (&m)[4], float am, const float (&v)[4],
                                                                 const float (&r)[4], float av_quick, float av_exact,
                                                                 Pack<1, 4>& mout, Pack<1, 4>& vout) {
     BothLane4 lane{m, am, v, r, av_quick, av_exact, mout, vout};
     HwWave<BothLane4> wave{lane};
-    requantize_both_verified<4>(wave);
+    requantize_both_verified<4, SCALED>(wave);
 }
 // Four elements per lane, one state (momentum kernels on fp32 parameters): plain conversion and byte packing.
 __device__ __forceinline__ void quantize_mom(const float (&m)[4], float am, Pack<1, 4>& out) {

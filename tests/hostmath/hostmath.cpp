@@ -185,16 +185,18 @@ void adam_tensor(void* mom, uint16_t* mom_scales, void* var, uint16_t* var_scale
                 } else {
                     adam_moments_plain(gr, in ? load_elem<DT>(mom, i) : 0.0f, in ? load_elem<DT>(var, i) : 0.0f, h, mn, vn);
                 }
-                const float rk = (QUANT || !EXACT) ? hw::sqrt(vn) : 0.0f;
+                float rk;
                 RedoLane<EPL>& R = redo[l];
-                R.p_old[k] = p0; R.m[k] = mn; R.v[k] = vn; r[l][k] = rk;
+                R.p_old[k] = p0; R.m[k] = mn; R.v[k] = vn;
                 if constexpr (EXACT) {
-                    R.p[k] = adam_apply_exact(DECOUPLED ? p0 * h.one_m_wd : p0, mn, vn, h);
+                    R.p[k] = adam_apply_exact(DECOUPLED ? p0 * h.one_m_wd : p0, mn, vn, h, rk);
                     R.slack[k] = 0.0f;
                 } else {
+                    rk = hw::sqrt(vn);
                     R.p[k] = adam_apply_folded<DECOUPLED>(p0, mn, rk, h, AdamFoldedGuard<DT, ECCB>::value, R.slack[k]);
                     if (flagged && in && adam_folded_is_flagged(R.slack[k])) ++*flagged;
                 }
+                r[l][k] = rk;
                 lane_am[l] = fmaxf(lane_am[l], fabsf(mn));
                 lane_vmax[l] = fmaxf(lane_vmax[l], vn);
             }
@@ -211,6 +213,7 @@ void adam_tensor(void* mom, uint16_t* mom_scales, void* var, uint16_t* var_scale
         if (QUANT) {
             float am[kLanes], av_quick[kLanes], av[kLanes];
             group_scales<EPL>(lane_am, lane_vmax, am, av_quick, av);
+            if (EXACT) for (float& a : av_quick) a *= h.rcp_sqrt_bc2;
             if constexpr (EPL == 8) {
                 for (int l = 0; l < kLanes; ++l) {
                     ml[l].am = am[l]; vl[l].av_quick = av_quick[l]; vl[l].av = av[l];
@@ -219,14 +222,14 @@ void adam_tensor(void* mom, uint16_t* mom_scales, void* var, uint16_t* var_scale
                 SimWave<MomLane<EPL>> mw{ml};
                 SimWave<VarLane<EPL>> vw{vl};
                 requantize_mom_verified<EPL>(mw);
-                requantize_var_verified<EPL>(vw);
+                requantize_var_verified<EPL, EXACT>(vw);
             } else {
                 for (int l = 0; l < kLanes; ++l) {
                     bl[l].am = am[l]; bl[l].av_quick = av_quick[l]; bl[l].av = av[l];
                     for (int k = 0; k < EPL; ++k) { bl[l].m[k] = redo[l].m[k]; bl[l].v[k] = redo[l].v[k]; bl[l].r[k] = r[l][k]; }
                 }
                 SimWave<BothLane<EPL>> bw{bl};
-                requantize_both_verified<EPL>(bw);
+                requantize_both_verified<EPL, EXACT>(bw);
             }
             for (int l = 0; l < kLanes; ++l) {
                 const int64_t first = base + (int64_t)l * EPL;

@@ -516,6 +516,25 @@ def test_extreme_learning_rates_and_eps(lr, eps):
             parity.check_master(a["p"], a["e"], b["p"], b["e"], f"lr {lr:g} eps {eps:g} step {step}")
 
 
+@pytest.mark.parametrize("noise", [0, 7])
+@pytest.mark.parametrize("dtype,ecc_dtype", [(torch.float32, None), (torch.bfloat16, torch.int16)])
+def test_second_moment_codes_from_the_updates_root(noise, dtype, ecc_dtype):
+    """The operation-by-operation kernels requantise the second moment from sqrt(v / bc2).  From both sides of the largest
+    root the quick form takes (2^48) and bias corrections from 2^-24 (beta2 next to one) to 1, every bit equals the
+    oracle's; with beta2 = 1 (bc2 = 0, the update a NaN) codes and scales still do."""
+    H.set_noise(noise)
+    n = 4096 + 17
+    for beta2, step in ((1 - 2.0 ** -24, 1), (0.999, 1), (0.999, 100), (0.5, 40), (1.0, 3)):
+        for scale in (1e-18, 1e-3, 1e13, 1e15, 1e17):  # the largest square stays finite
+            a = _adam_state(n, dtype, ecc_dtype, True, seed=4)
+            g = (_rand(n, scale, 20 + step) * torch.exp2(torch.arange(n) % 11 - 5.0)).to(dtype)
+            b = _clone(a)
+            T.adam_step_ref(T.MomentState(b["m"], b["ms"]), T.MomentState(b["v"], b["vs"]), b["p"], g, b["e"], 1e-3, 0.9, beta2, 1e-8, 1e-5, True, step)
+            H.adam_step(a["m"], a["ms"], a["v"], a["vs"], a["p"], g, a["e"], 1e-3, 0.9, beta2, 1e-8, 1e-5, True, step)
+            for key in ("m", "ms", "v", "vs") + (() if beta2 == 1.0 else ("p", "e")):
+                assert a[key] is None or parity.bits_equal(a[key], b[key]), (beta2, step, scale, key)
+
+
 MOM_MODES = {
     "lion": dict(lr=1e-4, mom_coef=0.99, update_coef=0.9, weight_decay=0.1 * 1e-4, do_lion=True),
     "sgd": dict(lr=1e-2, mom_coef=0.9, update_coef=0.9, weight_decay=1e-4),

@@ -94,9 +94,13 @@ class FlashAdam(FlashOptimizer):
         return "exp_avg", "exp_avg_sq"
 
     def _advance_step(self, param_state: dict[str, Any]) -> Optional[int]:
-        step = None if _hostscan.advance is None else _hostscan.advance(param_state["step"])
-        if step is not None:
-            return int(step)
+        counter = param_state["step"]
+        # the helper answers for any number of equal counters; a parameter's own is one number, and the torch calls
+        # below refuse anything else
+        if _hostscan.advance is not None and isinstance(counter, torch.Tensor) and counter.dim() == 0:
+            step = _hostscan.advance(counter)
+            if step is not None:
+                return int(step)
         param_state["step"] += 1
         return int(param_state["step"].item())
 

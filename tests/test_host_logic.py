@@ -511,3 +511,12 @@ def test_hostscan_step_args_declines_what_is_not_on_a_gpu():
     assert _hostscan.step_args(p, None, None, None, None, None, None, False) is None
     with pytest.raises(TypeError):
         _hostscan.step_args(p)
+
+
+@pytest.mark.parametrize("n", [0, 2, 3])
+def test_a_step_counter_that_is_not_one_number_is_refused(n):
+    opt = object.__new__(FlashAdamW)  # the counter alone; a whole optimizer needs a GPU
+    with pytest.raises(RuntimeError):
+        opt._advance_step({"step": torch.zeros(n)})
+    state = {"step": torch.tensor(6.0)}
+    assert opt._advance_step(state) == 7 and state["step"].item() == 7.0

@@ -773,7 +773,7 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
                     if error_bits is not None:
                         state["error_bits"] = error_bits
                         continue
-                batch.launch_if_reading(local_param)
+                batch.order_import(local_value, local_param)
                 local_param.copy_(local_value.to(param.dtype))
                 if "error_bits" in state:
                     width = local_param.element_size() + state["error_bits"].element_size()

@@ -160,7 +160,7 @@ class ConversionBatch:
         self._jobs: dict = {}  # (entry point, *its leading arguments, device) -> flat list of fo_convert_job words
         self._keepalive: list = []  # inputs must outlive the launch
         self._import_sources: set = set()  # storages that pending imports read
-        self._import_targets: set = set()  # storages and addresses that pending imports write
+        self._import_targets: dict = {}  # storages that pending imports write -> first and end address written in each
 
     def _add(self, entry: tuple, device: torch.device, src: torch.Tensor, src2, dst: torch.Tensor, dst2, flags: int = 0) -> None:
         ptr = _native.ptr
@@ -220,13 +220,13 @@ class ConversionBatch:
         out = torch.empty(narrow.shape, dtype=torch.int8 if width == 1 else torch.int16, device=narrow.device)
         if narrow.numel() == 0:
             return out
-        source, target = x.untyped_storage().data_ptr(), narrow.untyped_storage().data_ptr()
-        if source == target:
+        if x.untyped_storage().data_ptr() == narrow.untyped_storage().data_ptr():
             return None
-        if source in self._import_targets or target in self._import_sources or ("at", narrow.data_ptr()) in self._import_targets:
-            self.launch()  # tensors that share memory keep the order of the calls; jobs of one launch have none
-        self._import_sources.add(source)
-        self._import_targets.update((target, ("at", narrow.data_ptr())))
+        self.order_import(x, narrow)
+        self._import_sources.add(x.untyped_storage().data_ptr())
+        target, first, end = _span(narrow)
+        lo, hi = self._import_targets.get(target, (first, end))
+        self._import_targets[target] = (min(lo, first), max(hi, end))
         self._add(("fo_ecc_narrow_many", DTYPE_CODE[narrow.dtype], width), narrow.device, x, None, narrow, out)
         return out
 
@@ -251,10 +251,28 @@ class ConversionBatch:
         self._import_sources.clear()
         self._import_targets.clear()
 
-    def launch_if_reading(self, t: torch.Tensor) -> None:
-        """``launch()`` if a pending import reads the memory of `t`, which is about to be written."""
-        if self._import_sources and t.untyped_storage().data_ptr() in self._import_sources:
+    def order_import(self, value: torch.Tensor, param: torch.Tensor) -> None:
+        """``launch()`` if a pending import writes the memory of `value`, or reads or writes that of `param`: tensors that
+        share memory keep the order of the calls, and jobs of one launch have none.  Parameters carved from one buffer
+        one after the other share a launch: what counts is the span written in that buffer so far."""
+        if not self._import_targets:
+            return
+        if not type(value) is type(param) is torch.Tensor:  # whose memory cannot be asked for
             self.launch()
+            return
+        target, first, end = _span(param)
+        lo, hi = self._import_targets.get(target, (0, 0))
+        if (value.untyped_storage().data_ptr() in self._import_targets or target in self._import_sources
+                or (first < hi and lo < end)):
+            self.launch()
+
+
+def _span(t: torch.Tensor) -> tuple[int, int, int]:
+    """Address of the storage, first and end address of the elements of a tensor (strides are never negative)."""
+    extent = t.numel()
+    if extent and not t.is_contiguous():
+        extent = 1 + sum((size - 1) * stride for size, stride in zip(t.shape, t.stride()))
+    return t.untyped_storage().data_ptr(), t.data_ptr(), t.data_ptr() + extent * t.element_size()
 
 
 # ------------------------------------------------------------------------------------------------- ECC

@@ -207,3 +207,27 @@ def test_imports_that_share_memory_keep_their_order():
     assert (m.a == 2.0).all() and (m.b == 2.0).all() and (m.c == 9.0).all()
     opt.set_fp32_model_state_dict(m, {"b": m.c.data, "c": torch.full((n,), 4.0, device=DEV)})
     assert (m.b == 9.0).all() and (m.c == 4.0).all()
+
+
+def test_imports_into_overlapping_spans_keep_their_order():
+    """Two parameters that overlap in one buffer: the later import wins where they do, by the one-pass kernel and by the
+    general path (a value that is not contiguous); and a value that lives in a parameter imported before it."""
+    import flashoptim_amd as fo
+
+    n, shift = 6000, 2048
+    flat = torch.zeros(n + shift, device=DEV, dtype=torch.bfloat16)
+    m = torch.nn.Module()
+    m.a, m.b = torch.nn.Parameter(flat[:n]), torch.nn.Parameter(flat[shift:])
+    m.c, m.d = torch.nn.Parameter(torch.zeros(n, device=DEV, dtype=torch.bfloat16)), torch.nn.Parameter(torch.zeros(n // 2, device=DEV))
+    opt = fo.FlashAdamW(m.parameters(), lr=1e-3)
+    for p in m.parameters():
+        p.grad = torch.zeros_like(p)
+        opt.step_param(p)  # one after the other: a and b overlap
+    value = lambda v: torch.full((n,), v, device=DEV)  # noqa: E731
+    for late in (value(2.0), torch.full((2 * n,), 2.0, device=DEV)[::2]):
+        opt.set_fp32_model_state_dict(m, {"a": value(1.0), "b": late})
+        assert (flat[:shift] == 1.0).all() and (flat[shift:] == 2.0).all()
+    words = torch.zeros(n // 2, device=DEV)  # c's memory read as 32-bit words is d's value
+    m.c.data = words.view(torch.bfloat16)
+    opt.set_fp32_model_state_dict(m, {"c": value(5.0), "d": words})
+    assert (m.c == 5.0).all() and torch.equal(m.d.data, m.c.data.view(torch.float32))

@@ -1,7 +1,7 @@
 """Loader of the optional C++ helper that validates cached launch plans (flashoptim_amd/hostscan/fo_hostscan.cpp).
 
-Its functions (``scan``, ``same_objects``, ``counters``, ``advance``, ``step_args``) are None when the module has not been built (``make -C flashoptim_amd/hostscan``) or
-was built against another torch: the optimizer then walks its parameters in Python, 0.25 us per parameter instead of
+Its functions (``scan``, ``same_objects``, ``counters``, ``advance``, ``step_args``) are None when the module has not been
+built (``make -C flashoptim_amd/hostscan``) or was built against another torch: the optimizer then walks its parameters in Python, 0.25 us per parameter instead of
 0.06.  Host-side bookkeeping only; the step itself has no fallback (flashoptim_amd/_native.py).
 ``FLASHOPTIM_NO_HOSTSCAN=1`` keeps the Python walk.
 """

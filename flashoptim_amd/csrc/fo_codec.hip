@@ -104,9 +104,9 @@ template <int DT> __device__ __forceinline__ float one_nan(float x) { return (DT
 
 // ref:2541-2607 _triton_dequantize_kernel, with the cast to the output type that follows it in a checkpoint (ref:167).
 // Bound by memory: 1.06 bytes in and 4 (fp32) or 2 (bf16) out per element.  kSpans: the 1 KiB table that a workgroup
-// copies to LDS serves 1024 elements; reading the table through the vector cache instead is slower by a third.  An AdamW checkpoint of 2.2e8 weights (bf16, 24-bit
-// masters; this kernel and Int8WidenOp) takes 307 us, 6.5 TB/s, where fp32 values, their casts and torch's int8 cast
-// (1.3 TB/s) took 1456.
+// copies to LDS serves 1024 elements; reading the table through the vector cache instead is slower by a third.  An AdamW
+// checkpoint of 2.2e8 weights (bf16, 24-bit masters; this kernel and Int8WidenOp) takes 306 us, 6.5 TB/s, where fp32
+// values, their casts and torch's int8 cast (1.3 TB/s) took 1453.
 template <int ODT> struct DequantizeOp {
     static constexpr int kEpl = DTypeInfo<ODT>::epl, kSpans = ODT == DT_F32 ? 4 : 2, kLutFloats = 256;
     struct Raw { Pack<1, kEpl> codes; uint16_t scale; };

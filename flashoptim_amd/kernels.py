@@ -10,6 +10,7 @@ All of them are asynchronous on the current stream of the tensors' device and mu
 from __future__ import annotations
 
 import ctypes
+from bisect import bisect_left, bisect_right
 from typing import Optional
 
 import torch
@@ -148,6 +149,32 @@ def _codec_flags(signed: bool, sqrt: bool, softsign: bool) -> int:  # fo_codec_f
     return (1 if signed else 0) | (2 if sqrt else 0) | (4 if softsign else 0)
 
 
+class _Spans:
+    """A set of addresses, held as disjoint spans in ascending order."""
+
+    def __init__(self) -> None:
+        self._first: list = []
+        self._end: list = []
+
+    def meets(self, first: int, end: int) -> bool:
+        i = bisect_right(self._first, first)
+        return (i > 0 and self._end[i - 1] > first) or (i < len(self._first) and self._first[i] < end)
+
+    def add(self, first: int, end: int) -> None:
+        lo, hi = bisect_left(self._end, first), bisect_right(self._first, end)  # the spans it overlaps or touches
+        if lo < hi:
+            first, end = min(first, self._first[lo]), max(end, self._end[hi - 1])
+        self._first[lo:hi], self._end[lo:hi] = [first], [end]
+
+
+def _span(t: torch.Tensor) -> tuple[int, int]:
+    """First and end address of the elements of a tensor (strides are never negative)."""
+    extent = t.numel()
+    if extent and not t.is_contiguous():
+        extent = 1 + sum((size - 1) * stride for size, stride in zip(t.shape, t.stride()))
+    return t.data_ptr(), t.data_ptr() + extent * t.element_size()
+
+
 class ConversionBatch:
     """Conversions of many tensors, issued as one launch per kind, dtype and device (up to 64 tensors each) instead of
     one or two launches per tensor.
@@ -159,8 +186,10 @@ class ConversionBatch:
     def __init__(self) -> None:
         self._jobs: dict = {}  # (entry point, *its leading arguments, device) -> flat list of fo_convert_job words
         self._keepalive: list = []  # inputs must outlive the launch
-        self._import_sources: set = set()  # storages that pending imports read
-        self._import_targets: dict = {}  # storages that pending imports write -> first and end address written in each
+        # memory that pending imports read and write: addresses, since one memory can belong to several storage objects
+        # (dlpack, tensors of other libraries)
+        self._import_sources, self._import_targets = _Spans(), _Spans()
+        self._importing = False
 
     def _add(self, entry: tuple, device: torch.device, src: torch.Tensor, src2, dst: torch.Tensor, dst2, flags: int = 0) -> None:
         ptr = _native.ptr
@@ -220,13 +249,13 @@ class ConversionBatch:
         out = torch.empty(narrow.shape, dtype=torch.int8 if width == 1 else torch.int16, device=narrow.device)
         if narrow.numel() == 0:
             return out
-        if x.untyped_storage().data_ptr() == narrow.untyped_storage().data_ptr():
+        source, target = _span(x), _span(narrow)
+        if source[0] < target[1] and target[0] < source[1]:
             return None
         self.order_import(x, narrow)
-        self._import_sources.add(x.untyped_storage().data_ptr())
-        target, first, end = _span(narrow)
-        lo, hi = self._import_targets.get(target, (first, end))
-        self._import_targets[target] = (min(lo, first), max(hi, end))
+        self._import_sources.add(*source)
+        self._import_targets.add(*target)
+        self._importing = True
         self._add(("fo_ecc_narrow_many", DTYPE_CODE[narrow.dtype], width), narrow.device, x, None, narrow, out)
         return out
 
@@ -248,31 +277,22 @@ class ConversionBatch:
                 rc = getattr(_native.lib(), name)(table, len(words) // 6, *args, _native.current_stream_ptr(device))
             _native.check(rc, name)
         self._keepalive.clear()
-        self._import_sources.clear()
-        self._import_targets.clear()
+        if self._importing:
+            self._import_sources, self._import_targets = _Spans(), _Spans()
+            self._importing = False
 
     def order_import(self, value: torch.Tensor, param: torch.Tensor) -> None:
         """``launch()`` if a pending import writes the memory of `value`, or reads or writes that of `param`: tensors that
         share memory keep the order of the calls, and jobs of one launch have none.  Parameters carved from one buffer
-        one after the other share a launch: what counts is the span written in that buffer so far."""
-        if not self._import_targets:
+        side by side share a launch."""
+        if not self._importing:
             return
         if not type(value) is type(param) is torch.Tensor:  # whose memory cannot be asked for
             self.launch()
             return
-        target, first, end = _span(param)
-        lo, hi = self._import_targets.get(target, (0, 0))
-        if (value.untyped_storage().data_ptr() in self._import_targets or target in self._import_sources
-                or (first < hi and lo < end)):
+        target = _span(param)
+        if self._import_targets.meets(*_span(value)) or self._import_targets.meets(*target) or self._import_sources.meets(*target):
             self.launch()
-
-
-def _span(t: torch.Tensor) -> tuple[int, int, int]:
-    """Address of the storage, first and end address of the elements of a tensor (strides are never negative)."""
-    extent = t.numel()
-    if extent and not t.is_contiguous():
-        extent = 1 + sum((size - 1) * stride for size, stride in zip(t.shape, t.stride()))
-    return t.untyped_storage().data_ptr(), t.data_ptr(), t.data_ptr() + extent * t.element_size()
 
 
 # ------------------------------------------------------------------------------------------------- ECC

@@ -4,6 +4,7 @@ check_numerics' closed form, cast_model and the argument checks of gradient rele
 import ctypes
 import math
 import os
+import random
 import re
 from collections import OrderedDict
 
@@ -520,3 +521,70 @@ def test_a_step_counter_that_is_not_one_number_is_refused(n):
         opt._advance_step({"step": torch.zeros(n)})
     state = {"step": torch.tensor(6.0)}
     assert opt._advance_step(state) == 7 and state["step"].item() == 7.0
+
+
+# --------------------------------------------------------------------------------------- order of fp32 imports
+
+
+class _ImportOrder:
+    """A ConversionBatch over CPU tensors that says they are on the GPU; its launches are counted instead of issued."""
+
+    def __init__(self, monkeypatch):
+        from flashoptim_amd.kernels import ConversionBatch
+
+        monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+        self.launches = 0
+        self.batch = ConversionBatch()
+        issue = self.batch.launch
+
+        def launch():
+            self.launches += bool(self.batch._jobs)
+            self.batch._jobs = {}  # nothing reaches the device
+            issue()
+
+        monkeypatch.setattr(self.batch, "launch", launch)
+
+    def add(self, value, param):
+        """The import of `value` into `param`; whether it had to wait for a launch of those before it."""
+        before = self.launches
+        assert self.batch.import_fp32(value, param, torch.empty(param.shape, dtype=torch.int8)) is not None
+        return self.launches > before
+
+
+def _other_storage(t):
+    """The same memory as another storage object, whose address is the tensor's own."""
+    return torch.from_dlpack(t)
+
+
+@pytest.mark.parametrize("alias", [lambda t: t, _other_storage])
+def test_imports_that_overlap_in_memory_wait_for_each_other(alias, monkeypatch):
+    order = _ImportOrder(monkeypatch)
+    n = 6000
+    flat, value = torch.zeros(3 * n, dtype=torch.bfloat16), torch.zeros(n)
+    assert not order.add(value, flat[:n])
+    assert not order.add(value, alias(flat[2 * n:]))   # beside it
+    assert not order.add(value, alias(flat[n:2 * n]))  # between the two: touches both, overlaps neither
+    assert order.add(value, alias(flat[n - 1:2 * n - 1]))
+    words = torch.zeros(n)
+    param = words.view(torch.bfloat16)
+    assert not order.add(torch.zeros(2 * n), param)
+    assert order.add(alias(words[n // 2:]), torch.zeros(n // 2, dtype=torch.bfloat16))  # reads what is written
+    assert not order.add(words[:n // 2], torch.zeros(n // 2, dtype=torch.bfloat16))
+    assert not order.add(words[5:], torch.zeros(n - 5, dtype=torch.bfloat16))           # reads may overlap
+    assert order.add(value[:3], alias(param[3:6]))                                      # writes what is read
+
+
+@pytest.mark.parametrize("alias", [lambda t: t, _other_storage])
+def test_an_import_that_reads_its_own_target_is_declined(alias, monkeypatch):
+    order = _ImportOrder(monkeypatch)
+    words = torch.zeros(64)
+    target = words.view(torch.bfloat16)[96:]  # the upper half of what is read
+    assert order.batch.import_fp32(alias(words[32:]), target, torch.empty(32, dtype=torch.int8)) is None
+
+
+def test_many_imports_into_one_buffer_share_a_launch(monkeypatch):
+    order = _ImportOrder(monkeypatch)
+    flat, value = torch.zeros(64 * 500, dtype=torch.bfloat16), torch.zeros(64)
+    places = list(range(500))
+    random.Random(0).shuffle(places)
+    assert not any([order.add(value, flat[64 * i:64 * i + 64]) for i in places])

@@ -766,6 +766,7 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
                 local_param = self._get_local_tensor(param.data)
                 local_value = self._get_local_tensor(value)
                 if local_value.device != local_param.device:
+                    batch.order_import(local_value, local_param)  # it may live in a parameter whose import is pending
                     local_value = local_value.to(local_param.device)
                 state = self.state.get(param, {})
                 if "error_bits" in state:

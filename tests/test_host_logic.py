@@ -588,3 +588,28 @@ def test_many_imports_into_one_buffer_share_a_launch(monkeypatch):
     places = list(range(500))
     random.Random(0).shuffle(places)
     assert not any([order.add(value, flat[64 * i:64 * i + 64]) for i in places])
+
+
+def test_a_value_on_another_device_is_copied_after_the_imports_it_may_have_to_wait_for(monkeypatch):
+    """The copy reads the value's memory: a pending import into it has to be issued first."""
+    from flashoptim_amd import kernels
+
+    events = []
+
+    class Elsewhere:  # a value on another GPU
+        dtype, device = torch.float32, torch.device("cuda", 1)
+
+        def to_local(self):
+            return self
+
+        def to(self, device):
+            events.append("copied")
+            return torch.ones(8)
+
+    monkeypatch.setattr(kernels.ConversionBatch, "order_import", lambda self, value, param: events.append(type(value).__name__))
+    opt = object.__new__(FlashAdamW)
+    opt.state, opt._plan_epoch = {}, 0
+    model = nn.Module()
+    model.w = nn.Parameter(torch.zeros(8, dtype=torch.bfloat16))
+    opt.set_fp32_model_state_dict(model, {"w": Elsewhere()})
+    assert events[:2] == ["Elsewhere", "copied"] and (model.w == 1).all()

@@ -706,8 +706,9 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
             self._state_ready = set()
             return
         opt_state = cast(dict[torch.Tensor, Any], state["state"])
-        # one launch for the conversions of all parameters, as in state_dict()
-        batch = kernels.ConversionBatch()
+        # one launch for the conversions of all parameters, as in state_dict(), or several where the values are copies that
+        # torch made of the checkpoint's
+        batch = kernels.ConversionBatch(lasting=self._checkpoint_tensors)
         shared = {"batch": batch} if type(self)._load_state_for_param is FlashOptimizer._load_state_for_param else {}
         for group in cast(list[dict[str, Any]], state["param_groups"]):
             for param in group["params"]:
@@ -725,9 +726,19 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
         self._group_cache = {}
         self._state_ready = set()
 
+    # id()s of the tensors of the checkpoint that is being loaded: what torch hands on of it unchanged is no copy
+    _checkpoint_tensors: Any = frozenset()
+
     def load_state_dict(self, state_dict: dict[str, Any]) -> None:
         """Also accepts checkpoints of the stock torch optimizers, which may lack ``initial_lr`` (ref:974-986)."""
-        super().load_state_dict(state_dict)
+        try:
+            self._checkpoint_tensors = {id(v) for entry in state_dict["state"].values() for v in entry.values()}
+        except (AttributeError, KeyError, TypeError):
+            pass  # super() says what is wrong with it
+        try:
+            super().load_state_dict(state_dict)
+        finally:
+            self._checkpoint_tensors = frozenset()
         for group in self.param_groups:
             group.setdefault("initial_lr", group["lr"])
 
@@ -767,7 +778,7 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
                 local_value = self._get_local_tensor(value)
                 if local_value.device != local_param.device:
                     batch.order_import(local_value, local_param)  # it may live in a parameter whose import is pending
-                    local_value = local_value.to(local_param.device)
+                    local_value = batch.hold_copy(local_value.to(local_param.device))
                 state = self.state.get(param, {})
                 if "error_bits" in state:
                     error_bits = batch.import_fp32(local_value, local_param, state["error_bits"])

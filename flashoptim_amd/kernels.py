@@ -175,15 +175,26 @@ def _span(t: torch.Tensor) -> tuple[int, int]:
     return t.data_ptr(), t.data_ptr() + extent * t.element_size()
 
 
+# Bytes of copies (a host value's device copy, a checkpoint's cast values) that a ConversionBatch keeps alive before it
+# launches what it has: such a list would otherwise need the memory of all its copies at once.  A launch over this much takes
+# 70 us and more, beside which its own cost of a few us does not count, least of all next to the copies.
+_COPIES_HELD = 256 << 20
+
+
 class ConversionBatch:
     """Conversions of many tensors, issued as one launch per kind, dtype and device (up to 64 tensors each) instead of
     one or two launches per tensor.
 
     A method allocates its output and returns it at once; the values are there, in stream order, after ``launch()``.
     A batch is used by one thread, inside one call of this package.
+
+    ``lasting``: the id()s of the inputs that outlive the batch; others are copies that nobody else holds.  None: every
+    input outlives it, but for those a caller names (``hold_copy``).
     """
 
-    def __init__(self) -> None:
+    def __init__(self, lasting: Optional[set] = None) -> None:
+        self._lasting = lasting
+        self._copied = 0  # bytes of the copies it keeps alive
         self._jobs: dict = {}  # (entry point, *its leading arguments, device) -> flat list of fo_convert_job words
         self._keepalive: list = []  # inputs must outlive the launch
         # memory that pending imports read and write: addresses, since one memory can belong to several storage objects
@@ -196,11 +207,24 @@ class ConversionBatch:
         self._jobs.setdefault((entry, device), []).extend(
             (src.data_ptr(), ptr(src2) or 0, dst.data_ptr(), ptr(dst2) or 0, dst.numel(), flags))
         self._keepalive.append((src, src2, dst, dst2))
+        if self._copied >= _COPIES_HELD:
+            self.launch()
+
+    def hold_copy(self, t: torch.Tensor) -> torch.Tensor:
+        """`t`, an input that is freed with the launch."""
+        self._copied += t.numel() * t.element_size()
+        return t
+
+    def _input(self, t: torch.Tensor) -> torch.Tensor:
+        """`t` as the kernels read it."""
+        if not t.is_contiguous():
+            return self.hold_copy(t.contiguous())
+        return t if self._lasting is None or id(t) in self._lasting else self.hold_copy(t)
 
     def dequantize_bf16(self, codes: torch.Tensor, scales: torch.Tensor, signed: bool, sqrt: bool, softsign: bool) -> torch.Tensor:
         """``dequantize(codes, scales, ...).to(torch.bfloat16)``."""
         _check_codes(codes, scales, signed)
-        codes, scales = codes.contiguous(), scales.contiguous()
+        codes, scales = self._input(codes), self._input(scales)
         out = torch.empty_like(codes, dtype=torch.bfloat16)
         if codes.numel() > 0:
             self._add(("fo_dequantize_many", DTYPE_CODE[torch.bfloat16]), codes.device, codes, scales, out, None,
@@ -220,7 +244,7 @@ class ConversionBatch:
     def quantize(self, x: torch.Tensor, signed: bool, sqrt: bool, softsign: bool) -> tuple[torch.Tensor, torch.Tensor]:
         """:func:`quantize` of one tensor."""
         _check_values(x)
-        x = x.contiguous()
+        x = self._input(x)
         n = x.numel()
         codes = torch.empty_like(x, dtype=torch.int8 if signed else torch.uint8)
         scales = torch.empty((n + GROUP_SIZE - 1) // GROUP_SIZE, device=x.device, dtype=torch.float16)
@@ -235,7 +259,7 @@ class ConversionBatch:
             return values.to(dtype=torch.int8)
         out = torch.empty_like(values, dtype=torch.int8)
         if values.numel() > 0:
-            self._add(("fo_int8_narrow_many", DTYPE_CODE[values.dtype]), values.device, values, None, out, None)
+            self._add(("fo_int8_narrow_many", DTYPE_CODE[values.dtype]), values.device, self._input(values), None, out, None)
         return out
 
     def import_fp32(self, x: torch.Tensor, narrow: torch.Tensor, error_bits: torch.Tensor) -> Optional[torch.Tensor]:
@@ -265,7 +289,7 @@ class ConversionBatch:
         out = torch.empty(param.shape, dtype=torch.float32, device=param.device)
         if param.numel() > 0:
             self._add(("fo_ecc_join_many", DTYPE_CODE[param.dtype], error_bits.element_size()), param.device,
-                      param.contiguous(), error_bits.contiguous(), out, None)
+                      self._input(param), self._input(error_bits), out, None)
         return out
 
     def launch(self) -> None:
@@ -277,6 +301,7 @@ class ConversionBatch:
                 rc = getattr(_native.lib(), name)(table, len(words) // 6, *args, _native.current_stream_ptr(device))
             _native.check(rc, name)
         self._keepalive.clear()
+        self._copied = 0
         if self._importing:
             self._import_sources, self._import_targets = _Spans(), _Spans()
             self._importing = False

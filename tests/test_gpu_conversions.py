@@ -231,3 +231,67 @@ def test_imports_into_overlapping_spans_keep_their_order():
     m.c.data = words.view(torch.bfloat16)
     opt.set_fp32_model_state_dict(m, {"c": value(5.0), "d": words})
     assert (m.c == 5.0).all() and torch.equal(m.d.data, m.c.data.view(torch.float32))
+
+
+def _peak_above_start(call):
+    torch.cuda.synchronize()
+    start = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    call()
+    torch.cuda.synchronize()
+    return torch.cuda.max_memory_allocated() - start
+
+
+def _stepped(n_tensors, n, dtype, **kw):
+    import flashoptim_amd as fo
+
+    m = torch.nn.ParameterList([torch.nn.Parameter(torch.randn(n, device=DEV).to(dtype)) for _ in range(n_tensors)])
+    opt = fo.FlashAdamW(m.parameters(), lr=1e-3, **kw)
+    for p in m:
+        p.grad = torch.randn_like(p)
+    opt.step()
+    return m, opt
+
+
+def test_import_of_host_masters_holds_few_of_them_on_the_device(monkeypatch):
+    """The device copies of a list of host tensors do not add up: beside the new correction codes at most the batch's
+    budget and the value at hand are alive."""
+    from flashoptim_amd import kernels
+
+    budget = 8 << 20
+    monkeypatch.setattr(kernels, "_COPIES_HELD", budget, raising=False)
+    n_tensors, n = 24, 1 << 20
+    m, opt = _stepped(n_tensors, n, torch.bfloat16)
+    masters = {k: torch.randn(n) for k, _ in m.named_parameters()}
+    peak = _peak_above_start(lambda: opt.set_fp32_model_state_dict(m, masters))
+    # the new codes (the launch plan of the last step keeps the old ones), the copies, the value at hand
+    assert peak <= n_tensors * n + budget + 4 * n, peak
+    for k, p in m.named_parameters():
+        want = masters[k].to(torch.bfloat16)
+        assert torch.equal(p.detach().cpu(), want), k
+        assert torch.equal(opt.state[p]["error_bits"], kernels.compute_ecc_bits(masters[k].to(DEV), p.detach(), 3)), k
+
+
+@pytest.mark.parametrize("compress", [False, True])
+def test_load_of_a_host_checkpoint_frees_what_it_has_converted(compress, monkeypatch):
+    """torch brings the whole checkpoint to the device in the parameters' dtype first; each part is freed once it is
+    converted, give or take the batch's budget.  A checkpoint on the device stays whole in one launch."""
+    from flashoptim_amd import kernels
+
+    budget = 8 << 20
+    monkeypatch.setattr(kernels, "_COPIES_HELD", budget, raising=False)
+    n_tensors, n = 24, 1 << 20
+    m, opt = _stepped(n_tensors, n, torch.bfloat16, compress_state_dict=compress)
+    saved = opt.state_dict()
+    host = {"state": {i: {k: v.cpu() if isinstance(v, torch.Tensor) else v for k, v in st.items()} for i, st in saved["state"].items()},
+            "param_groups": saved["param_groups"]}
+    cast = 6 * n_tensors * n  # both moments and the correction codes, two bytes each
+    peak = _peak_above_start(lambda: opt.load_state_dict(host))
+    assert peak <= cast + cast // 32 + budget + 8 * n, peak
+    states = lambda: [t for p in m for st in [opt.state[p]] for t in (  # noqa: E731
+        st["exp_avg"].quantized, st["exp_avg"].scales, st["exp_avg_sq"].quantized, st["exp_avg_sq"].scales, st["error_bits"])]
+    loaded, launches, issue = states(), [], kernels.ConversionBatch.launch
+    monkeypatch.setattr(kernels.ConversionBatch, "launch", lambda self: (launches.append(len(self._jobs)), issue(self)))
+    opt.load_state_dict(saved)
+    assert len(launches) == 1
+    assert all(torch.equal(a, b) for a, b in zip(loaded, states()))

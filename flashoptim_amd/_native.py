@@ -95,6 +95,7 @@ DIAG_SIGNATURES = {
     "fo_adam_step_residency": (_i32, [_i32] * 5 + [_vp] * 3),
     "fo_momentum_step_residency": (_i32, [_i32] * 5 + [_vp] * 3),
     "fo_probe_residency": (_i32, [_i32, _vp, _i64, _vp, _vp]),
+    "fo_conversion_launch": (_i32, [_vp, _i64, _i64, _i64, _vp]),
 }
 
 

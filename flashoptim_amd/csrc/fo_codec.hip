@@ -11,6 +11,9 @@
 #include "fo_device.h"
 #include "fo_host.h"
 #include "../../include/flashoptim_hip.h"
+#ifdef FO_DIAG
+#include "../../include/flashoptim_hip_diag.h"
+#endif
 
 namespace fo {
 
@@ -346,38 +349,57 @@ __global__ __launch_bounds__(kCodecThreads) void ecc_split_kernel(const float* x
 namespace {
 using namespace fo_host;
 
+// A launch takes fewer than 2^32 work-items.
+constexpr int64_t kMaxBlocks = UINT32_MAX / fo::kCodecThreads;
+
 // One short-lived workgroup per span of 64 x EPL elements (one pass streams better than a persistent grid here).
 unsigned grid_for(int64_t n, int epl) {
     const int64_t spans = (n + 64 * epl - 1) / (64 * epl);
-    return (unsigned)(spans < INT32_MAX ? spans : INT32_MAX);
+    return (unsigned)(spans < kMaxBlocks ? spans : kMaxBlocks);
 }
 
 int32_t codec_flags(int is_signed, int do_sqrt, int softsign) {
     return (is_signed ? FO_CODEC_SIGNED : 0) | (do_sqrt ? FO_CODEC_SQRT : 0) | (softsign ? FO_CODEC_SOFTSIGN : 0);
 }
 
+// One launch's share of a job list: the jobs before `end` that have elements, and the workgroups they take together.
+struct JobRange { int64_t end, blocks; };
+
+// The jobs from `first` on that share a launch, at `per_block` elements to a workgroup; no job takes more than kMaxBlocks.
+JobRange jobs_of_launch(const fo_convert_job* jobs, int64_t n_jobs, int64_t first, int64_t per_block) {
+    JobRange r{first, 0};
+    for (int count = 0; r.end < n_jobs; ++r.end) {
+        const int64_t need = (jobs[r.end].n + per_block - 1) / per_block;
+        if (need == 0) continue;
+        if (count == fo::kJobsPerLaunch || r.blocks + need > kMaxBlocks) break;
+        ++count;
+        r.blocks += need;
+    }
+    return r;
+}
+
 // Enqueues the jobs, kJobsPerLaunch to a launch; the caller has checked their pointers.
 template <class Op> int launch_jobs(const fo_convert_job* jobs, int64_t n_jobs, hipStream_t stream) {
-    fo::JobBatch b;
-    b.count = 0; b.reserved = 0;
-    int64_t blocks = 0;
-    const auto flush = [&]() -> int {
-        if (b.count == 0) return 0;
-        hipLaunchKernelGGL(fo::convert_kernel<Op>, dim3((unsigned)blocks), dim3(fo::kCodecThreads), 0, stream, b);
-        b.count = 0; blocks = 0;
-        return check_hip(hipGetLastError(), "conversion kernel launch");
-    };
-    for (int64_t i = 0; i < n_jobs; ++i) {
-        if (jobs[i].n == 0) continue;
-        const int64_t need = (jobs[i].n + fo::ConvertShape<Op>::kBlock - 1) / fo::ConvertShape<Op>::kBlock;
-        if (need > INT32_MAX) return fail(FO_ERR_INVALID_ARGUMENT, "tensor too large for one launch (%lld elements)", (long long)jobs[i].n);
-        if (b.count == fo::kJobsPerLaunch || blocks + need > INT32_MAX)
-            if (int rc = flush()) return rc;
-        b.job[b.count] = jobs[i];
-        b.first_block[b.count++] = (fo::u32)blocks;
-        blocks += need;
+    constexpr int64_t kBlock = fo::ConvertShape<Op>::kBlock;
+    for (int64_t i = 0; i < n_jobs; ++i)
+        if (jobs[i].n > kMaxBlocks * kBlock)
+            return fail(FO_ERR_INVALID_ARGUMENT, "tensor too large for one launch (%lld elements, at most %lld)", (long long)jobs[i].n, (long long)(kMaxBlocks * kBlock));
+    for (int64_t first = 0; first < n_jobs;) {
+        const JobRange r = jobs_of_launch(jobs, n_jobs, first, kBlock);
+        fo::JobBatch b;
+        b.count = 0; b.reserved = 0;
+        fo::u32 block = 0;
+        for (; first < r.end; ++first) {
+            if (jobs[first].n == 0) continue;
+            b.job[b.count] = jobs[first];
+            b.first_block[b.count++] = block;
+            block += (fo::u32)((jobs[first].n + kBlock - 1) / kBlock);
+        }
+        if (r.blocks == 0) continue;
+        hipLaunchKernelGGL(fo::convert_kernel<Op>, dim3((unsigned)r.blocks), dim3(fo::kCodecThreads), 0, stream, b);
+        if (int rc = check_hip(hipGetLastError(), "conversion kernel launch")) return rc;
     }
-    return flush();
+    return 0;
 }
 
 // What every job list has to satisfy before a kernel sees its pointers: src, dst (and src2, dst2 where the kernel uses
@@ -509,5 +531,13 @@ int fo_ecc_narrow_many(const fo_convert_job* jobs, int64_t n_jobs, int narrow_dt
     if (int rc = validate_jobs(jobs, n_jobs, 4, 0, 2, (unsigned)ecc_bytes)) return rc;
     FO_ECC_JOBS(EccNarrowOp)
 }
+
+#ifdef FO_DIAG
+int fo_conversion_launch(const fo_convert_job* jobs, int64_t n_jobs, int64_t first, int64_t elements_per_workgroup, int64_t* workgroups) {
+    const JobRange r = jobs_of_launch(jobs, n_jobs, first, elements_per_workgroup);
+    if (workgroups) *workgroups = r.blocks;
+    return (int)(r.end - first);
+}
+#endif  // FO_DIAG
 
 }  // extern "C"

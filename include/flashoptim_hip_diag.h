@@ -62,6 +62,14 @@ int fo_momentum_step_residency(int dtype, int ecc_bytes, int quantized, int kind
  */
 int fo_probe_residency(int dynamic_lds_bytes, void *counters, int64_t counters_bytes, int *most_resident, void *stream);
 
+/*
+ * How a list of conversions (flashoptim_hip.h: fo_convert_job) is split into launches; nothing is launched and only the
+ * jobs' `n` is read.  Returns how many jobs from `first` on the launch that starts there covers, empty ones included;
+ * `workgroups` receives the size of its grid.
+ */
+int fo_conversion_launch(const fo_convert_job *jobs, int64_t n_jobs, int64_t first, int64_t elements_per_workgroup,
+                         int64_t *workgroups);
+
 #ifdef __cplusplus
 }
 #endif

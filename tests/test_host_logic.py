@@ -613,3 +613,28 @@ def test_a_value_on_another_device_is_copied_after_the_imports_it_may_have_to_wa
     model.w = nn.Parameter(torch.zeros(8, dtype=torch.bfloat16))
     opt.set_fp32_model_state_dict(model, {"w": Elsewhere()})
     assert events[:2] == ["Elsewhere", "copied"] and (model.w == 1).all()
+
+
+def test_conversion_lists_are_split_below_the_largest_grid():
+    """A launch takes fewer than 2^32 work-items, 64 to a workgroup, and at most 64 tensors; every job is launched once."""
+    diag, top = _native.diag_lib(), (2 ** 32 - 1) // 64
+
+    def launches(lengths, per_block):
+        jobs = (ctypes.c_int64 * (6 * len(lengths)))(*[w for n in lengths for w in (0, 0, 0, 0, n, 0)])
+        first, out, blocks = 0, [], ctypes.c_int64()
+        while first < len(lengths):
+            taken = diag.fo_conversion_launch(jobs, len(lengths), first, per_block, ctypes.byref(blocks))
+            part = [-(-n // per_block) for n in lengths[first:first + taken] if n]
+            assert taken > 0 and sum(part) == blocks.value <= top and len(part) <= 64
+            out.append(taken)
+            first += taken
+        assert first == len(lengths)
+        return out
+
+    block = 512
+    assert launches([top * block], block) == [1]
+    assert launches([top * block - 1, 0, 1, 5], block) == [2, 2]    # one workgroup too many
+    assert launches([block * (top - 1), 3, 0], block) == [3]
+    assert launches([1 << 33] * 5, block) == [3, 2]                 # 2^24 workgroups each: four would be 2^26
+    assert launches([7] * 130 + [0] * 70, block) == [64, 64, 72]
+    assert launches([0] * 100, block) == [100]

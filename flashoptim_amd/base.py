@@ -482,11 +482,10 @@ class FlashOptimizer(torch.optim.Optimizer, abc.ABC):
                 # the counters are live state the caller may have rewritten (a warm restart zeroes them): take the
                 # step number from them, and leave counters that no longer agree to the per-parameter path.  A
                 # counter OBJECT that was replaced (state[p]["step"] = tensor(0.)) no longer aliases the pool.
+                lo = None
                 if _hostscan.counters is not None:
                     lo = _hostscan.counters(self.state, b.params, b.step_views, b.step_pool)
-                    if lo is None:
-                        return False
-                else:
+                if lo is None:  # changed, or states in mappings the C++ walk does not look into
                     state = self.state
                     if [id(state[p].get("step")) for p in b.params] != b.step_view_ids:
                         return False

@@ -638,3 +638,37 @@ def test_conversion_lists_are_split_below_the_largest_grid():
     assert launches([1 << 33] * 5, block) == [3, 2]                 # 2^24 workgroups each: four would be 2^26
     assert launches([7] * 130 + [0] * 70, block) == [64, 64, 72]
     assert launches([0] * 100, block) == [100]
+
+
+@pytest.mark.parametrize("entry", [dict, OrderedDict])
+@pytest.mark.parametrize("state", [dict, OrderedDict, type("Checked", (dict,), {"__getitem__": lambda self, key: dict.__getitem__(self, key)})])
+def test_a_cached_plan_serves_states_kept_in_other_mappings(state, entry, monkeypatch):
+    """What the C++ walk over the counters does not vouch for goes through the Python one, which says whether the plan
+    holds; only counters that were really replaced or differ send the group back to planning."""
+    from types import SimpleNamespace
+
+    from flashoptim_amd import _hostscan
+    from flashoptim_amd.base import _Bucket, _GroupCache
+
+    monkeypatch.setattr(_hostscan, "scan", None)
+    params = [nn.Parameter(torch.zeros(4)) for _ in range(3)]
+    for p in params:
+        p.grad = torch.ones(4)
+    pool = torch.full((3,), 6.0)
+    views = [pool[i] for i in range(3)]
+    opt = object.__new__(FlashAdamW)
+    opt.state, opt._decoupled, opt._exact_update = state(), False, False
+    for p, v in zip(params, views):
+        opt.state[p] = entry(step=v)
+    steps = []
+    plan = SimpleNamespace(grad_ptrs=[p.grad.data_ptr() for p in params], param_ptrs=[p.data_ptr() for p in params],
+                           launch=lambda **scalars: steps.append(scalars["step"]))
+    bucket = _Bucket("adam", torch.float32, 0, True, params, [], plan, pool, 6, views, list(map(id, views)))
+    cache = _GroupCache(0, params, list(map(id, params)), "adam", [bucket], [], 3)
+    group = dict(lr=1e-3, betas=(0.9, 0.999), eps=1e-8, weight_decay=0.0)
+    assert opt._step_group_fast(cache, group) and steps == [7] and pool.tolist() == [7.0] * 3
+    opt.state[params[1]]["step"] = torch.tensor(7.0)
+    assert not opt._step_group_fast(cache, group)
+    opt.state[params[1]]["step"] = views[1]
+    pool[2] = 8.0
+    assert not opt._step_group_fast(cache, group) and steps == [7]

@@ -175,6 +175,12 @@ def _span(t: torch.Tensor) -> tuple[int, int]:
     return t.data_ptr(), t.data_ptr() + extent * t.element_size()
 
 
+def _as_stored(t: torch.Tensor) -> bool:
+    """Whether the memory of a tensor holds its elements in order and as they are: no subclass, no strides, no negation that
+    torch has put off."""
+    return type(t) is torch.Tensor and t.is_contiguous() and not t.is_neg()
+
+
 # Bytes of copies (a host value's device copy, a checkpoint's cast values) that a ConversionBatch keeps alive before it
 # launches what it has: such a list would otherwise need the memory of all its copies at once.  A launch over this much takes
 # 70 us and more, beside which its own cost of a few us does not count, least of all next to the copies.
@@ -233,8 +239,7 @@ class ConversionBatch:
 
     def widen_int8(self, values: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
         """``values.to(dtype)`` of an int8 tensor, dtype bf16 or fp16."""
-        if (type(values) is not torch.Tensor or not values.is_cuda or values.dtype != torch.int8
-                or not values.is_contiguous() or dtype not in (torch.bfloat16, torch.float16)):
+        if not _as_stored(values) or not values.is_cuda or values.dtype != torch.int8 or dtype not in (torch.bfloat16, torch.float16):
             return values.to(dtype=dtype)
         out = torch.empty_like(values, dtype=dtype)
         if values.numel() > 0:
@@ -254,8 +259,7 @@ class ConversionBatch:
 
     def narrow_to_int8(self, values: torch.Tensor) -> torch.Tensor:
         """``values.to(torch.int8)`` of a bf16 or fp16 tensor."""
-        if (type(values) is not torch.Tensor or not values.is_cuda or not values.is_contiguous()
-                or values.dtype not in (torch.bfloat16, torch.float16)):
+        if not _as_stored(values) or not values.is_cuda or values.dtype not in (torch.bfloat16, torch.float16):
             return values.to(dtype=torch.int8)
         out = torch.empty_like(values, dtype=torch.int8)
         if values.numel() > 0:
@@ -265,8 +269,8 @@ class ConversionBatch:
     def import_fp32(self, x: torch.Tensor, narrow: torch.Tensor, error_bits: torch.Tensor) -> Optional[torch.Tensor]:
         """``narrow.copy_(x)`` and the new correction term ``compute_ecc_bits(x, narrow, ...)`` of `error_bits`' width in
         one pass; None (and nothing done) where the tensors are not laid out for it."""
-        if (not type(x) is type(narrow) is torch.Tensor or x.dtype != torch.float32 or x.shape != narrow.shape
-                or not x.is_contiguous() or not narrow.is_contiguous() or not narrow.is_cuda or x.device != narrow.device
+        if (not _as_stored(x) or not _as_stored(narrow) or x.dtype != torch.float32 or x.shape != narrow.shape
+                or not narrow.is_cuda or x.device != narrow.device
                 or narrow.dtype not in (torch.bfloat16, torch.float16) or error_bits.element_size() not in (1, 2)):
             return None
         width = error_bits.element_size()
@@ -371,7 +375,7 @@ def compute_ecc_bits(
     )
     n = narrow_param.numel()
     if n > 0:
-        x = fp32_param.to(narrow_param.device).contiguous()
+        x = fp32_param.to(narrow_param.device).resolve_neg().contiguous()
         narrow = narrow_param.contiguous()
         with _native.device_guard(narrow.device):
             rc = _native.lib().fo_ecc_split(

@@ -295,3 +295,22 @@ def test_load_of_a_host_checkpoint_frees_what_it_has_converted(compress, monkeyp
     opt.load_state_dict(saved)
     assert len(launches) == 1
     assert all(torch.equal(a, b) for a, b in zip(loaded, states()))
+
+
+def test_values_with_a_negation_put_off_are_converted_as_what_they_stand_for():
+    import flashoptim_amd as fo
+    from flashoptim_amd.kernels import ConversionBatch, compute_ecc_bits
+
+    m = torch.nn.Module()
+    m.w = torch.nn.Parameter(torch.zeros(700, device=DEV, dtype=torch.bfloat16))
+    opt = fo.FlashAdamW(m.parameters(), lr=1e-3)
+    m.w.grad = torch.zeros_like(m.w)
+    opt.step()
+    master = torch.randn(700, device=DEV)
+    opt.set_fp32_model_state_dict(m, {"w": torch._neg_view(master)})
+    assert torch.equal(m.w.detach(), (-master).to(torch.bfloat16))
+    assert torch.equal(opt.state[m.w]["error_bits"], compute_ecc_bits(-master, m.w.detach(), 3))
+    batch, codes = ConversionBatch(), torch.arange(-100, 100, device=DEV, dtype=torch.int8)
+    narrow, wide = batch.narrow_to_int8(torch._neg_view(codes.to(torch.bfloat16))), batch.widen_int8(torch._neg_view(codes), torch.bfloat16)
+    batch.launch()
+    assert torch.equal(narrow, -codes) and torch.equal(wide, -codes.to(torch.bfloat16))

@@ -127,10 +127,16 @@ PyObject* same_objects(PyObject*, PyObject* args) {
 }
 
 // dict[key] as a borrowed reference (nullptr: absent, or an error that is cleared).  A tensor's hash is its id(), evaluated
-// by a Python function; `by_address` says that the caller has seen this hold for a key of the same type.
+// by a Python function; `by_address` says that the caller has seen this hold for a key of the same type.  The lookup that
+// takes a known hash is in CPython's headers up to 3.12.
 PyObject* find(PyObject* dict, PyObject* key, bool by_address) {
+#if PY_VERSION_HEX < 0x030d0000
     const Py_hash_t hash = by_address ? (Py_hash_t)(uintptr_t)key : PyObject_Hash(key);
     PyObject* value = hash == -1 ? nullptr : _PyDict_GetItem_KnownHash(dict, key, hash);
+#else
+    (void)by_address;
+    PyObject* value = PyDict_GetItemWithError(dict, key);
+#endif
     if (!value) PyErr_Clear();
     return value;
 }

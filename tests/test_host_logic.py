@@ -672,3 +672,37 @@ def test_a_cached_plan_serves_states_kept_in_other_mappings(state, entry, monkey
     opt.state[params[1]]["step"] = views[1]
     pool[2] = 8.0
     assert not opt._step_group_fast(cache, group) and steps == [7]
+
+
+# ----------------------------------------------------------------------------------------------------- build
+
+
+def test_a_failing_build_step_shows_its_first_error():
+    import sys
+
+    import __graft_entry__ as entry
+
+    noise = "print('note: ' + 'x' * 70);" * 200
+    with pytest.raises(RuntimeError, match="(?s)status 3.*a.hip:7: error: no such thing"):
+        entry._run([sys.executable, "-c", f"{noise}print('a.hip:7: error: no such thing');{noise}import sys;sys.exit(3)"])
+
+
+def test_the_build_goes_on_without_the_host_helper(monkeypatch):
+    import __graft_entry__ as entry
+    from flashoptim_amd import _hostscan
+
+    ran = []
+
+    def run(cmd):
+        ran.append(" ".join(cmd))
+        if "hostscan" in ran[-1]:
+            raise RuntimeError("no headers")
+
+    monkeypatch.setattr(entry, "_run", run)
+    removed = []
+    monkeypatch.setattr(entry.os, "remove", removed.append)
+    monkeypatch.setattr(_hostscan, "scan", None)
+    with pytest.warns(UserWarning) as caught:
+        entry.build()
+    assert len(ran) == 5 and all(any(text in str(w.message) for w in caught) for text in ("no headers", "does not load"))
+    assert removed == [_hostscan.library_path()]  # no helper of older sources stays behind

@@ -137,8 +137,6 @@ __device__ __forceinline__ void store_scale(uint16_t* scales, Where w, uint16_t 
 __device__ __forceinline__ uint16_t load_scale(const uint16_t* scales, Where w) {
     return ((const FO_GLOBAL uint16_t*)(scales + (w.span >> 5)))[(unsigned)(w.lane >> 5)];
 }
-// per-lane 64-bit group index (cold kernels)
-__device__ __forceinline__ void store_scale(uint16_t* scales, int64_t group, uint16_t bits) { ((FO_GLOBAL uint16_t*)scales)[group] = bits; }
 
 // Guarded path (tensor tails, unaligned views): element-wise accesses, out-of-range elements read as zero and
 // are never written (ref:1625-1630, 2296-2301 masked loads with other=0).

@@ -7,8 +7,8 @@
 // Nothing here touches memory, lanes or LDS.  fp32 throughout; the translation units are compiled with
 // -ffp-contract=off, so a fused multiply-add happens only where fmaf() is written.
 //
-// The kernels lean on four hardware approximations (v_rcp_f32, v_rsq_f32, v_sqrt_f32: within one ulp, correctly
-// rounded for 85-90 % of inputs on MI355X) and on a few exact instructions (v_ldexp_f32, v_med3, v_cvt_flr).
+// The kernels lean on three hardware approximations (v_rcp_f32, v_rsq_f32, v_sqrt_f32: within one ulp, correctly
+// rounded for 85-90 % of inputs on MI355X) and on a few exact instructions (v_med3, v_fract, v_cvt_flr).
 // In the host build they are stand-ins with the same contract; `fo_math_host_noise` != 0 makes the approximate
 // ones err by an ulp in a pseudo-random direction, which is how the CPU tests show that every result that
 // is meant to be correctly rounded stays so whatever the hardware returns inside its error bound.
@@ -72,7 +72,6 @@ static inline float rcp(float x) { return nudge((float)(1.0 / (double)x), x); }
 static inline float rsq(float x) { return nudge((float)(1.0 / sqrt((double)x)), x); }
 static inline float sqrt(float x) { return nudge(sqrtf(x), x); }
 static inline float fract(float x) { return x - floorf(x); }
-static inline float ldexp(float x, int e) { return ldexpf(x, e); }
 static inline float med3(float x, float lo, float hi) { return fminf(fmaxf(x, lo), hi); }
 static inline int floor_to_int(float x) { return (int)floorf(x); }
 static inline float fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
@@ -81,7 +80,6 @@ FO_FN float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 FO_FN float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
 FO_FN float sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 FO_FN float fract(float x) { return __builtin_amdgcn_fractf(x); }  // x - floor(x)
-FO_FN float ldexp(float x, int e) { return __builtin_amdgcn_ldexpf(x, e); }
 FO_FN float med3(float x, float lo, float hi) { return __builtin_amdgcn_fmed3f(x, lo, hi); }
 // (int)floor(x) in one instruction
 FO_FN int floor_to_int(float x) {
@@ -257,13 +255,13 @@ FO_FN u32 quantize_var_code(float r, float av, float rav) { return (u32)(int)qua
 // 2^-24 relative, each approximate instruction at most an ulp; in code units, with |x| <= 128 resp. 256):
 //     first moment   exact 3.8e-5, quick 3.8e-5   ->  they can differ by 7.6e-5   ->  margin 2^-13 = 1.2e-4
 //     second moment  exact 7.6e-5, quick 1.2e-4   ->  they can differ by 2.0e-4   ->  margin 2^-12 = 2.4e-4
+// so when the quick value lies farther than the margin from every integer, floor() of it IS the exact form's code.
 // The operation-by-operation Adam update has a root at hand, of v / bc2 (a quotient, correctly rounded, and a corrected
 // root: 1.5u with u = 2^-24).  The quick form takes it in place of hw::sqrt(v), whose instruction costs four issue slots,
 // and av / sqrt(bc2) (two roundings more, 2u) in place of av: 9.5u instead of 8u on a value up to 256, 1.45e-4 for the
 // quick form, 2.2e-4 together.  v / bc2 must not overflow for that, so a group whose largest root reaches kQuickLargestVar
 // takes the exact form (bc2, one minus an fp32 power, is zero or at least 2^-24; where it is zero every root is a NaN,
 // which fails the test too).
-// so when the quick value lies farther than the margin from every integer, floor() of it IS the exact form's code.
 // Precondition: am + |m| and av stay below 2^126 (beyond that the reciprocal instruction returns a subnormal, flushed
 // to zero).  The group scale is stored as fp16 and overflows at 65504, forty orders of magnitude earlier, so a state
 // that large is already lost; the bound is stated, not enforced.

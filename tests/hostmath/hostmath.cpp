@@ -3,7 +3,7 @@
 // This file compiles flashoptim_amd/csrc/fo_math.h -- the very functions the gfx950 kernels call per element --
 // for the host and wraps them in loops that mirror the kernels' structure (quantisation groups of 32 elements,
 // masked tail elements read as zero, group maxima, code packing).  The instructions the kernels take from the
-// hardware (reciprocal, reciprocal root, ldexp, floor-convert, the narrowing conversions) are stand-ins with the
+// hardware (reciprocal, reciprocal root, floor-convert, the narrowing conversions) are stand-ins with the
 // same contract; fo_math_host_noise != 0 makes the approximate ones err by an ulp.  The tests compare the
 // output with the independent IEEE restatement of the reference in oracle/, without a GPU.
 //

@@ -73,7 +73,8 @@ static inline float rsq(float x) { return nudge((float)(1.0 / sqrt((double)x)), 
 static inline float sqrt(float x) { return nudge(sqrtf(x), x); }
 static inline float fract(float x) { return x - floorf(x); }
 static inline float med3(float x, float lo, float hi) { return fminf(fmaxf(x, lo), hi); }
-static inline int floor_to_int(float x) { return (int)floorf(x); }
+static inline int floor_to_int(float x) { return x == x ? (int)floorf(x) : -1; }
+static inline float minimum(float a, float b) { return a != a ? a : b != b ? b : fminf(a, b); }
 static inline float fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 #else
 FO_FN float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
@@ -81,12 +82,13 @@ FO_FN float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
 FO_FN float sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 FO_FN float fract(float x) { return __builtin_amdgcn_fractf(x); }  // x - floor(x)
 FO_FN float med3(float x, float lo, float hi) { return __builtin_amdgcn_fmed3f(x, lo, hi); }
-// (int)floor(x) in one instruction
+// (int)floor(x) in one instruction; -1 for a NaN, where a conversion that truncates gives 0
 FO_FN int floor_to_int(float x) {
     int r;
     asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
     return r;
 }
+FO_FN float minimum(float a, float b) { return __builtin_elementwise_minimum(a, b); }  // a NaN if either is; two of them are one v_minimum3_f32
 FO_FN float fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 #endif
 FO_FN u32 clamp_u32(u32 x, u32 lo, u32 hi) {  // one v_med3_u32
@@ -562,7 +564,8 @@ template <int N, bool SCALED = false, class Wave> FO_FN void requantize_both_ver
 // The standalone codec over a lane's N values of one kind (VAR: second moments).  Lane members:
 //   v[N], am            the values and what their group is divided by (codec_mom_code, codec_var_code)
 //   x[N], slack[N], least         scratch of the flow
-//   convert(x)          codes of all N values from their quick values
+//   convert(x)          codes of all N values from their quick values (anything for a NaN: the general form gives its
+//                       code, so `least` is a minimum that lets a NaN through)
 //   set_code(k, c)      replaces the code of position k
 template <int N, bool VAR, class Wave> FO_FN void codec_verified(Wave& wave) {
     constexpr float kMargin = VAR ? kQuickMarginVar : kQuickMarginMom;
@@ -573,7 +576,7 @@ template <int N, bool VAR, class Wave> FO_FN void codec_verified(Wave& wave) {
             L.slack[k] = quick_value_slack(L.x[k]);
         }
         L.least = L.slack[0];
-        FO_UNROLL for (int k = 1; k < N; ++k) L.least = fminf(L.least, L.slack[k]);
+        FO_UNROLL for (int k = 1; k < N; ++k) L.least = hw::minimum(L.least, L.slack[k]);
         L.convert(L.x);
     });
     if (wave.any([](const auto& L) FO_LANE_ATTR { return !(L.am < kCodecLargest) || !quick_slack_is_safe(L.least, kMargin); })) {

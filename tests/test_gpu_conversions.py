@@ -314,3 +314,42 @@ def test_values_with_a_negation_put_off_are_converted_as_what_they_stand_for():
     narrow, wide = batch.narrow_to_int8(torch._neg_view(codes.to(torch.bfloat16))), batch.widen_int8(torch._neg_view(codes), torch.bfloat16)
     batch.launch()
     assert torch.equal(narrow, -codes) and torch.equal(wide, -codes.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("second_moment", [False, True])
+def test_quantize_of_values_that_are_not_finite_or_negative(second_moment, dtype):
+    """The two kinds of state whose codes take a quick form, against the formula in IEEE arithmetic: NaN, infinities and
+    negative second moments (a NaN after the root), alone in a lane and beside ordinary values, at every place of it.  A NaN
+    takes no part in the group's maximum and its code is 0, what the conversion instruction makes of it."""
+    from flashoptim_amd.kernels import ConversionBatch
+
+    nan, inf = float("nan"), float("inf")
+    g = torch.Generator().manual_seed(11)
+    odd = [nan, -nan, inf, -inf, -1.0, -0.0, 1e-30]
+    rows = []
+    for value in odd:
+        for at in range(32):  # one of them at each place of a group
+            row = torch.randn(32, generator=g).abs()
+            row[at] = value
+            rows.append(row)
+        rows.append(torch.where(torch.arange(32) % 8 == 3, torch.randn(32, generator=g).abs(), torch.tensor(value)))
+        rows.append(torch.full((32,), value))
+    x = torch.cat(rows)
+    if not second_moment:
+        x = torch.where((torch.rand(x.shape, generator=g) < 0.5) & x.isfinite(), -x, x)
+    x = x.to(dtype)
+    batch = ConversionBatch()
+    codes, scales = batch.quantize(x.to(DEV), not second_moment, second_moment, not second_moment)
+    batch.launch()
+    v = x.float().view(-1, 32)
+    v = v.sqrt() if second_moment else v
+    top = v.abs().nan_to_num(0.0, posinf=inf).amax(1, keepdim=True).clamp(min=1e-12)
+    t = v / top
+    if second_moment:
+        q = (t * 255 + 0.5).floor()
+    else:
+        q = ((2 * t) / (1 + t.abs()) * 127 + 0.5).floor()
+    want = q.nan_to_num(0.0).to(torch.int32).view(-1).to(codes.dtype)
+    assert torch.equal(codes.cpu(), want)
+    assert parity.bits_equal(scales, top.view(-1).to(torch.float16))

@@ -152,6 +152,8 @@ def _codec_flags(signed: bool, sqrt: bool, softsign: bool) -> int:  # fo_codec_f
 class _Spans:
     """A set of addresses, held as disjoint spans in ascending order."""
 
+    __slots__ = ("_first", "_end")
+
     def __init__(self) -> None:
         self._first: list = []
         self._end: list = []
@@ -161,10 +163,14 @@ class _Spans:
         return (i > 0 and self._end[i - 1] > first) or (i < len(self._first) and self._first[i] < end)
 
     def add(self, first: int, end: int) -> None:
-        lo, hi = bisect_left(self._end, first), bisect_right(self._first, end)  # the spans it overlaps or touches
-        if lo < hi:
-            first, end = min(first, self._first[lo]), max(end, self._end[hi - 1])
-        self._first[lo:hi], self._end[lo:hi] = [first], [end]
+        starts, ends = self._first, self._end
+        i = bisect_right(starts, first)
+        if (i == 0 or ends[i - 1] <= first) and (i == len(starts) or starts[i] >= end):
+            starts.insert(i, first)
+            ends.insert(i, end)
+            return
+        lo, hi = bisect_right(ends, first), bisect_left(starts, end)  # the spans it overlaps
+        starts[lo:hi], ends[lo:hi] = [min(first, starts[lo])], [max(end, ends[hi - 1])]
 
 
 def _span(t: torch.Tensor) -> tuple[int, int]:
@@ -172,13 +178,8 @@ def _span(t: torch.Tensor) -> tuple[int, int]:
     extent = t.numel()
     if extent and not t.is_contiguous():
         extent = 1 + sum((size - 1) * stride for size, stride in zip(t.shape, t.stride()))
-    return t.data_ptr(), t.data_ptr() + extent * t.element_size()
-
-
-def _as_stored(t: torch.Tensor) -> bool:
-    """Whether the memory of a tensor holds its elements in order and as they are: no subclass, no strides, no negation that
-    torch has put off."""
-    return type(t) is torch.Tensor and t.is_contiguous() and not t.is_neg()
+    first = t.data_ptr()
+    return first, first + extent * t.element_size()
 
 
 # Bytes of copies (a host value's device copy, a checkpoint's cast values) that a ConversionBatch keeps alive before it
@@ -213,24 +214,22 @@ class ConversionBatch:
         self._jobs.setdefault((entry, device), []).extend(
             (src.data_ptr(), ptr(src2) or 0, dst.data_ptr(), ptr(dst2) or 0, dst.numel(), flags))
         self._keepalive.append((src, src2, dst, dst2))
-        if self._copied >= _COPIES_HELD:
-            self.launch()
 
     def hold_copy(self, t: torch.Tensor) -> torch.Tensor:
-        """`t`, an input that is freed with the launch."""
-        self._copied += t.numel() * t.element_size()
+        """`t`, the next input, which is freed with the launch."""
+        size = t.numel() * t.element_size()
+        if self._copied + size > _COPIES_HELD:
+            self.launch()
+        self._copied += size
         return t
 
-    def _input(self, t: torch.Tensor) -> torch.Tensor:
-        """`t` as the kernels read it."""
-        if not t.is_contiguous():
-            return self.hold_copy(t.contiguous())
-        return t if self._lasting is None or id(t) in self._lasting else self.hold_copy(t)
+    def _dense(self, t: torch.Tensor) -> torch.Tensor:
+        return t if t.is_contiguous() else self.hold_copy(t.contiguous())
 
     def dequantize_bf16(self, codes: torch.Tensor, scales: torch.Tensor, signed: bool, sqrt: bool, softsign: bool) -> torch.Tensor:
         """``dequantize(codes, scales, ...).to(torch.bfloat16)``."""
         _check_codes(codes, scales, signed)
-        codes, scales = self._input(codes), self._input(scales)
+        codes, scales = codes.contiguous(), scales.contiguous()  # a state's always are
         out = torch.empty_like(codes, dtype=torch.bfloat16)
         if codes.numel() > 0:
             self._add(("fo_dequantize_many", DTYPE_CODE[torch.bfloat16]), codes.device, codes, scales, out, None,
@@ -239,7 +238,8 @@ class ConversionBatch:
 
     def widen_int8(self, values: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
         """``values.to(dtype)`` of an int8 tensor, dtype bf16 or fp16."""
-        if not _as_stored(values) or not values.is_cuda or values.dtype != torch.int8 or dtype not in (torch.bfloat16, torch.float16):
+        if (type(values) is not torch.Tensor or not values.is_cuda or values.dtype != torch.int8 or values.is_neg()
+                or not values.is_contiguous() or dtype not in (torch.bfloat16, torch.float16)):
             return values.to(dtype=dtype)
         out = torch.empty_like(values, dtype=dtype)
         if values.numel() > 0:
@@ -249,7 +249,10 @@ class ConversionBatch:
     def quantize(self, x: torch.Tensor, signed: bool, sqrt: bool, softsign: bool) -> tuple[torch.Tensor, torch.Tensor]:
         """:func:`quantize` of one tensor."""
         _check_values(x)
-        x = self._input(x)
+        if not x.is_contiguous():
+            x = self.hold_copy(x.contiguous())
+        elif self._lasting is not None and id(x) not in self._lasting:
+            self.hold_copy(x)
         n = x.numel()
         codes = torch.empty_like(x, dtype=torch.int8 if signed else torch.uint8)
         scales = torch.empty((n + GROUP_SIZE - 1) // GROUP_SIZE, device=x.device, dtype=torch.float16)
@@ -259,30 +262,36 @@ class ConversionBatch:
 
     def narrow_to_int8(self, values: torch.Tensor) -> torch.Tensor:
         """``values.to(torch.int8)`` of a bf16 or fp16 tensor."""
-        if not _as_stored(values) or not values.is_cuda or values.dtype not in (torch.bfloat16, torch.float16):
+        if (type(values) is not torch.Tensor or not values.is_cuda or not values.is_contiguous() or values.is_neg()
+                or values.dtype not in (torch.bfloat16, torch.float16)):
             return values.to(dtype=torch.int8)
         out = torch.empty_like(values, dtype=torch.int8)
         if values.numel() > 0:
-            self._add(("fo_int8_narrow_many", DTYPE_CODE[values.dtype]), values.device, self._input(values), None, out, None)
+            if self._lasting is not None and id(values) not in self._lasting:
+                self.hold_copy(values)
+            self._add(("fo_int8_narrow_many", DTYPE_CODE[values.dtype]), values.device, values, None, out, None)
         return out
 
     def import_fp32(self, x: torch.Tensor, narrow: torch.Tensor, error_bits: torch.Tensor) -> Optional[torch.Tensor]:
         """``narrow.copy_(x)`` and the new correction term ``compute_ecc_bits(x, narrow, ...)`` of `error_bits`' width in
         one pass; None (and nothing done) where the tensors are not laid out for it."""
-        if (not _as_stored(x) or not _as_stored(narrow) or x.dtype != torch.float32 or x.shape != narrow.shape
-                or not narrow.is_cuda or x.device != narrow.device
-                or narrow.dtype not in (torch.bfloat16, torch.float16) or error_bits.element_size() not in (1, 2)):
+        if (not type(x) is type(narrow) is torch.Tensor or x.dtype != torch.float32 or x.shape != narrow.shape
+                or not x.is_contiguous() or not narrow.is_contiguous() or not narrow.is_cuda or x.device != narrow.device
+                or x.is_neg() or narrow.is_neg() or narrow.dtype not in (torch.bfloat16, torch.float16) or error_bits.element_size() not in (1, 2)):
             return None
         width = error_bits.element_size()
         out = torch.empty(narrow.shape, dtype=torch.int8 if width == 1 else torch.int16, device=narrow.device)
-        if narrow.numel() == 0:
+        n = narrow.numel()
+        if n == 0:
             return out
-        source, target = _span(x), _span(narrow)
-        if source[0] < target[1] and target[0] < source[1]:
+        source, target = x.data_ptr(), narrow.data_ptr()
+        source_end, target_end = source + 4 * n, target + 2 * n
+        if source < target_end and target < source_end:
             return None
-        self.order_import(x, narrow)
-        self._import_sources.add(*source)
-        self._import_targets.add(*target)
+        if self._importing:
+            self._order_spans(source, source_end, target, target_end)
+        self._import_sources.add(source, source_end)
+        self._import_targets.add(target, target_end)
         self._importing = True
         self._add(("fo_ecc_narrow_many", DTYPE_CODE[narrow.dtype], width), narrow.device, x, None, narrow, out)
         return out
@@ -293,7 +302,7 @@ class ConversionBatch:
         out = torch.empty(param.shape, dtype=torch.float32, device=param.device)
         if param.numel() > 0:
             self._add(("fo_ecc_join_many", DTYPE_CODE[param.dtype], error_bits.element_size()), param.device,
-                      self._input(param), self._input(error_bits), out, None)
+                      self._dense(param), self._dense(error_bits), out, None)
         return out
 
     def launch(self) -> None:
@@ -319,8 +328,11 @@ class ConversionBatch:
         if not type(value) is type(param) is torch.Tensor:  # whose memory cannot be asked for
             self.launch()
             return
-        target = _span(param)
-        if self._import_targets.meets(*_span(value)) or self._import_targets.meets(*target) or self._import_sources.meets(*target):
+        self._order_spans(*_span(value), *_span(param))
+
+    def _order_spans(self, source: int, source_end: int, target: int, target_end: int) -> None:
+        writes = self._import_targets
+        if writes.meets(target, target_end) or writes.meets(source, source_end) or self._import_sources.meets(target, target_end):
             self.launch()
 
 

@@ -58,15 +58,15 @@ static_assert(sizeof(JobBatch) <= 3584, "a batch must fit the kernel argument se
 // kSpans is each Op's best over five sets of 2^27 elements in turn (more than the caches hold), bf16 where the type is
 // free (TB/s of the bytes in and out):
 //     spans per workgroup         1      2      3      4      6      8
-//     fp32 masters out          6.01   6.54   6.33   6.42   6.14   6.34
-//     fp32 masters in           6.09   6.66   6.38   6.43   6.11   6.08
-//     dequantise to bf16        4.81   6.51   6.15   6.35   6.00   6.18
-//     dequantise to fp32        3.99   5.54   5.92   6.30   5.90   6.15
-//     quantise, first moments   4.20   6.08   6.07   6.28   5.92   6.02
-//     quantise, second moments  4.02   5.49   5.56   5.91   5.77   5.70
-//     quantise fp32             4.55   5.80   6.04   6.49   6.38   6.18
-//     int8 to bf16              5.28   6.56   6.16   6.24   6.13   6.17
-//     bf16 to int8              5.66   6.67   6.35   6.43   6.27   6.15
+//     fp32 masters out          6.02   6.62   6.28   6.35   6.12   6.27
+//     fp32 masters in           6.09   6.59   6.34   6.36   6.04   6.09
+//     dequantise to bf16        4.80   6.48   6.12   6.32   5.96   6.13
+//     dequantise to fp32        3.98   5.48   5.91   6.29   5.89   6.13
+//     quantise, first moments   4.22   6.02   6.03   6.20   5.86   5.94
+//     quantise, second moments  3.95   5.65   5.74   5.99   5.77   5.82
+//     quantise fp32             4.53   5.78   6.03   6.46   6.32   6.12
+//     int8 to bf16              5.25   6.48   6.14   6.17   6.04   6.15
+//     bf16 to int8              5.77   6.58   6.42   6.35   6.20   6.17
 // One span leaves what a workgroup costs to start (its place in the list, the table in LDS, the spread of its loads) over
 // too few bytes, many spans widen the window of addresses in flight; odd counts start workgroups at odd KiB.  A cap on the
 // resident workgroups gains nothing on top.

@@ -73,7 +73,7 @@ static inline float rsq(float x) { return nudge((float)(1.0 / sqrt((double)x)), 
 static inline float sqrt(float x) { return nudge(sqrtf(x), x); }
 static inline float fract(float x) { return x - floorf(x); }
 static inline float med3(float x, float lo, float hi) { return fminf(fmaxf(x, lo), hi); }
-static inline int floor_to_int(float x) { return x == x ? (int)floorf(x) : -1; }
+static inline int floor_to_int(float x) { return x == x ? (int)floorf(x) : INT32_MAX; }  // arithmetic makes positive NaNs there
 static inline float minimum(float a, float b) { return a != a ? a : b != b ? b : fminf(a, b); }
 static inline float fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 #else
@@ -82,7 +82,8 @@ FO_FN float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
 FO_FN float sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 FO_FN float fract(float x) { return __builtin_amdgcn_fractf(x); }  // x - floor(x)
 FO_FN float med3(float x, float lo, float hi) { return __builtin_amdgcn_fmed3f(x, lo, hi); }
-// (int)floor(x) in one instruction; -1 for a NaN, where a conversion that truncates gives 0
+// (int)floor(x) in one instruction; a NaN becomes the largest or the smallest int by its sign (low byte 255 or 0), where a
+// conversion that truncates gives 0
 FO_FN int floor_to_int(float x) {
     int r;
     asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
